@@ -233,6 +233,16 @@ typedef struct pe_rope_args {
    path (packed_encoders/ops.py:464-499). */
 int pe_rope_qkv_fwd(const pe_rope_args *args, hipStream_t stream);
 
+/* Bias-free LayerNorm of contiguous bf16 rows, with the residual add of an encoder layer folded
+   in: s = bf16(x + residual) (or x when residual is NULL), out = bf16((s - mean(s)) *
+   rsqrt(var(s) + eps) * weight), statistics in fp32. sum receives s and is given exactly when
+   residual is. Every pointer 16-byte aligned; cols a multiple of 8, at most
+   PE_LAYER_NORM_MAX_COLS (else PE_ATTN_EUNSUPPORTED). sum and out may not overlap each other or
+   an input. Replaces the reference's fused LayerNorm tail (packed_encoders/ops.py:38-319). */
+#define PE_LAYER_NORM_MAX_COLS 4096
+int pe_layer_norm_fwd(const void *x, const void *residual, const void *weight, void *sum, void *out, int64_t rows,
+                      int32_t cols, float eps, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

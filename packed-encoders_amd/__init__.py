@@ -17,7 +17,7 @@ repository root) is its importable alias.
 from __future__ import annotations
 
 from . import errors, workloads
-from . import _lib, attention_dispatch, hip_attention
+from . import _lib, attention_dispatch, hip_attention, hip_dense
 from . import batch, config, locate, state, staging, ops, pieces, forward, graph, runtime_attention, pack as _pack_module
 from .batch import PackedBatch
 from .errors import PackedEncodersError, UnsupportedTargetError, ValidationError

@@ -34,6 +34,7 @@ HIPCC_FLAGS = [
     # AGPR-resident accumulators would cost a v_accvgpr_read per element and per rescale
     "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
+EXTENSION = HERE / "_pe_torch.so"  # native launches for torch tensors (csrc/pe_torch.cpp)
 SOURCES = ["pe_attn_capi.hip"]
 PEAKS_SOURCES = ["pe_peaks.hip"]
 
@@ -66,22 +67,43 @@ def hipcc() -> str:
 
 
 def build_library(verbose: bool = False) -> Path:
-    """Compile the attention library ``libpe_attn.so`` and the peaks microbenchmarks
-    ``libpe_peaks.so`` (each an atomic replace); returns the attention library's path."""
-    _compile(SOURCES, LIBRARY, verbose)
-    _compile(PEAKS_SOURCES, PEAKS_LIBRARY, verbose)
+    """Compile the attention library ``libpe_attn.so``, the peaks microbenchmarks
+    ``libpe_peaks.so`` and the torch extension ``_pe_torch.so`` (each an atomic replace); returns
+    the attention library's path."""
+    _compile([hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", *(str(CSRC / s) for s in SOURCES)], LIBRARY, verbose)
+    _compile([hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", *(str(CSRC / s) for s in PEAKS_SOURCES)], PEAKS_LIBRARY, verbose)
+    _compile(_extension_command(), EXTENSION, verbose)
     return LIBRARY
 
 
-def _compile(sources: list[str], target: Path, verbose: bool) -> None:
+def _extension_command() -> list[str]:
+    """g++ on csrc/pe_torch.cpp: host code only, linked against torch and, beside it, the
+    attention library."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    rocm = Path(hipcc()).resolve().parent.parent
+    includes = [root / "include", root / "include" / "torch" / "csrc" / "api" / "include",
+                rocm / "include" if (rocm / "include" / "hip").is_dir() else Path("/opt/rocm/include"),
+                Path(sysconfig.get_paths()["include"])]
+    return ["g++", "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *(arg for d in includes for arg in ("-isystem", str(d))), str(CSRC / "pe_torch.cpp"),
+            f"-L{root / 'lib'}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+            f"-L{HERE}", "-lpe_attn", "-Wl,-rpath,$ORIGIN"]
+
+
+def _compile(command: list[str], target: Path, verbose: bool) -> None:
     tmp = target.with_name(f"{target.name}.tmp{os.getpid()}")
-    cmd = [hipcc(), *HIPCC_FLAGS, f"-I{INCLUDE}", *(str(CSRC / s) for s in sources), "-o", str(tmp)]
+    cmd = [*command, "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     noise = "packed-fp32-ops' is not a recognized feature"
     stderr = "\n".join(line for line in proc.stderr.splitlines() if noise not in line)
     if proc.returncode != 0:
         tmp.unlink(missing_ok=True)
-        raise RuntimeError(f"hipcc failed ({proc.returncode}):\n{' '.join(cmd)}\n{stderr}")
+        raise RuntimeError(f"{Path(cmd[0]).name} failed ({proc.returncode}):\n{' '.join(cmd)}\n{stderr}")
     if verbose and stderr.strip():
         print(stderr)
     os.replace(tmp, target)

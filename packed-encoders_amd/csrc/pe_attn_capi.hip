@@ -18,6 +18,7 @@
 #include "pe_attn_short.h"
 #include "pe_attn_tiled.h"
 #include "pe_attn_tiled_wide16.h"
+#include "pe_dense.h"
 #include "pe_rope.h"
 
 namespace pe {
@@ -405,6 +406,23 @@ int launch_rope(const pe::RopeParams &p, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
 }
 
+template <bool ADD>
+int launch_norm(const pe::NormParams &p, hipStream_t stream) {
+    const int64_t blocks = (p.rows + 3) / 4;
+    if (blocks > 0x7fffffffLL) return PE_ATTN_EUNSUPPORTED;
+    const dim3 grid((unsigned)blocks), block(256);
+    const int pieces = (p.cols / 8 + 63) / 64;  // 16-byte pieces per lane
+    if (pieces <= 1)
+        hipLaunchKernelGGL((pe::layer_norm_kernel<1, ADD>), grid, block, 0, stream, p);
+    else if (pieces <= 2)
+        hipLaunchKernelGGL((pe::layer_norm_kernel<2, ADD>), grid, block, 0, stream, p);
+    else if (pieces <= 4)
+        hipLaunchKernelGGL((pe::layer_norm_kernel<4, ADD>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((pe::layer_norm_kernel<8, ADD>), grid, block, 0, stream, p);
+    return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
 }  // namespace
 
 extern "C" {
@@ -576,6 +594,28 @@ int pe_rope_qkv_fwd(const pe_rope_args *a, hipStream_t stream) {
     if (a->head_dim == 64) return launch_rope<64>(p, stream);
     if (a->head_dim == 128) return launch_rope<128>(p, stream);
     return launch_rope<256>(p, stream);
+}
+
+int pe_layer_norm_fwd(const void *x, const void *residual, const void *weight, void *sum, void *out, int64_t rows,
+                      int32_t cols, float eps, hipStream_t stream) {
+    if (rows < 0 || cols < 1) return PE_ATTN_EINVAL;
+    if ((cols & 7) || cols > PE_LAYER_NORM_MAX_COLS) return PE_ATTN_EUNSUPPORTED;
+    if (rows == 0) return PE_ATTN_OK;
+    if (!x || !weight || !out || (residual != nullptr) != (sum != nullptr)) return PE_ATTN_EINVAL;
+    const void *ptrs[5] = {x, residual, weight, sum, out};
+    for (const void *p : ptrs)
+        if (!aligned16(p)) return PE_ATTN_EINVAL;
+    pe::NormParams p;
+    p.x = static_cast<const __bf16 *>(x);
+    p.res = static_cast<const __bf16 *>(residual);
+    p.w = static_cast<const __bf16 *>(weight);
+    p.sum = static_cast<__bf16 *>(sum);
+    p.out = static_cast<__bf16 *>(out);
+    p.rows = rows;
+    p.cols = cols;
+    p.inv_cols = 1.0f / (float)cols;
+    p.eps = eps;
+    return residual ? launch_norm<true>(p, stream) : launch_norm<false>(p, stream);
 }
 
 }  // extern "C"

@@ -1,0 +1,104 @@
+// Row-wise passes of an encoder layer around its attention and products (gfx950): LayerNorm with
+// the residual add folded in, bound by HBM: every tensor is read or written once, in 16-byte
+// pieces, everything else stays in registers.
+#pragma once
+
+#include "pe_attn_device.h"
+
+namespace pe {
+
+// ----------------------------------------------------------------------------- LayerNorm
+
+struct NormParams {
+    const __bf16 *x;    // [rows, cols], contiguous
+    const __bf16 *res;  // the residual added first, or NULL
+    const __bf16 *w;    // [cols]
+    __bf16 *sum;        // bf16(x + res) (written), only with a residual
+    __bf16 *out;        // LayerNorm(x + res) * w (written)
+    int64_t rows;
+    int32_t cols;  // a multiple of 8
+    float inv_cols;
+    float eps;
+};
+
+// Sum over the wave's 64 lanes, the same bits on every lane: rotations within 16 lanes (DPP row_ror
+// by 8, 4, 2, 1), then the 16- and 32-lane swaps.
+__device__ __forceinline__ float wave_sum(float x) {
+    auto ror = [](float v, auto n) {
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + decltype(n)::value, 0xf, 0xf, true));
+    };
+    x += ror(x, std::integral_constant<int, 8>{});
+    x += ror(x, std::integral_constant<int, 4>{});
+    x += ror(x, std::integral_constant<int, 2>{});
+    x += ror(x, std::integral_constant<int, 1>{});
+    const unsigned u = __builtin_bit_cast(unsigned, x);
+    const auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    x = __builtin_bit_cast(float, (unsigned)s16[0]) + __builtin_bit_cast(float, (unsigned)s16[1]);
+    const unsigned w = __builtin_bit_cast(unsigned, x);
+    const auto s32 = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+    return __builtin_bit_cast(float, (unsigned)s32[0]) + __builtin_bit_cast(float, (unsigned)s32[1]);
+}
+
+// One wave per row, NC 16-byte pieces per lane (piece c * 64 + lane), so a row's statistics never
+// leave the wave: no LDS, no barrier, and the mean and the squared deviations are taken from the
+// row held in registers. Statistics in fp32 over the bf16 values the row holds (the sum is rounded
+// to bf16 first, as the residual stream is stored). The mean adds x / cols, so that no finite row
+// overflows it. With the residual at 32,438 x 768: 31.4 us for 199 MB (6.3 TB/s), against 53.3 +
+// 24.3 us for torch's add and LayerNorm, which move the sum twice more.
+template <int NC, bool ADD>
+__global__ __launch_bounds__(256) void layer_norm_kernel(NormParams p) {
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + uniform(threadIdx.x >> 6);
+    if (row >= p.rows) return;
+    const int64_t base = row * p.cols;
+    const int pieces = p.cols >> 3;
+    bf16x8 v[NC], r[ADD ? NC : 1], w[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int i = c * 64 + lane;
+        v[c] = i < pieces ? ld_g16(p.x + base + 8 * i) : bf16x8{};
+        if constexpr (ADD) r[c] = i < pieces ? ld_g16(p.res + base + 8 * i) : bf16x8{};
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int i = c * 64 + lane;
+        w[c] = i < pieces ? ld_g16(p.w + 8 * i) : bf16x8{};
+    }
+    float mean = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if constexpr (ADD) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[c][j] = (__bf16)((float)v[c][j] + (float)r[c][j]);
+            const int i = c * 64 + lane;
+            if (i < pieces) *reinterpret_cast<bf16x8 *>(p.sum + base + 8 * i) = v[c];
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) mean = fmaf((float)v[c][j], p.inv_cols, mean);
+    }
+    mean = wave_sum(mean);
+    float var = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        float part = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float d = (float)v[c][j] - mean;
+            part = fmaf(d, d, part);
+        }
+        var += c * 64 + lane < pieces ? part : 0.0f;
+    }
+    var = wave_sum(var) * p.inv_cols;
+    const float rstd = rsqrtf(var + p.eps);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int i = c * 64 + lane;
+        bf16x8 y;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = (__bf16)(((float)v[c][j] - mean) * rstd * (float)w[c][j]);
+        if (i < pieces) *reinterpret_cast<bf16x8 *>(p.out + base + 8 * i) = y;
+    }
+}
+
+}  // namespace pe

@@ -6,10 +6,10 @@ Attention — the hot path — goes to the HIP kernels (``hip_attention``): ``at
 short or the tiled kernel on the device. ``"sdpa"`` is the reference's dependency-free dense
 fallback (ops.py:327-339), reached only when it is asked for.
 
-The rest of the layer (LayerNorm, the projections, GeGLU, RoPE) is outside this build's scope
-and runs as plain torch ops with Hugging Face ModernBERT's numerics: LayerNorm without bias,
-bias-free linears, ``gelu(input) * gate``, split-half RoPE applied in fp32 with tables rounded to
-the model dtype.
+The rest of the layer has Hugging Face ModernBERT's numerics: LayerNorm without bias, bias-free
+linears, ``gelu(input) * gate``, split-half RoPE applied in fp32 with tables rounded to the model
+dtype. The linears are torch's; LayerNorm (with the residual add) and RoPE run on HIP kernels
+for bf16 inference (``hip_dense``, ``hip_attention.rope_qkv``) and as plain torch ops otherwise.
 """
 
 from __future__ import annotations
@@ -18,6 +18,8 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor
 
+from . import hip_dense
+
 BACKENDS = ("hip", "sdpa", "auto")
 
 
@@ -25,11 +27,15 @@ BACKENDS = ("hip", "sdpa", "auto")
 
 
 def layer_norm(x: Tensor, weight: Tensor, eps: float) -> Tensor:
-    return F.layer_norm(x, (x.shape[-1],), weight, None, eps)
+    out = hip_dense.layer_norm(x, weight, eps)
+    return F.layer_norm(x, (x.shape[-1],), weight, None, eps) if out is None else out
 
 
 def add_layer_norm(x: Tensor, residual: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     """``(x + residual, LayerNorm(x + residual))``: the residual stream and the next input."""
+    out = hip_dense.add_layer_norm(x, residual, weight, eps)
+    if out is not None:
+        return out
     summed = x + residual
     return summed, layer_norm(summed, weight, eps)
 
