@@ -243,6 +243,12 @@ int pe_rope_qkv_fwd(const pe_rope_args *args, hipStream_t stream);
 int pe_layer_norm_fwd(const void *x, const void *residual, const void *weight, void *sum, void *out, int64_t rows,
                       int32_t cols, float eps, hipStream_t stream);
 
+/* out [rows, width] = bf16(gelu(proj[:, :width]) * proj[:, width:]) of contiguous bf16 proj
+   [rows, 2 * width], the exact (normal distribution) gelu in fp32, rounded once. Pointers 16-byte
+   aligned, width a multiple of 8 (else PE_ATTN_EUNSUPPORTED); out may not overlap proj.
+   Replaces the reference's fused GeGLU (packed_encoders/ops.py:38-319). */
+int pe_geglu_fwd(const void *proj, void *out, int64_t rows, int32_t width, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -34,6 +34,7 @@ EXPORTED = (
     "pe_attn_kernels",
     "pe_rope_qkv_fwd",
     "pe_layer_norm_fwd",
+    "pe_geglu_fwd",
 )
 
 
@@ -142,6 +143,8 @@ def library(path: str | None = None) -> ctypes.CDLL:
     lib.pe_layer_norm_fwd.restype = ctypes.c_int
     lib.pe_layer_norm_fwd.argtypes = [*[ctypes.c_void_p] * 5, ctypes.c_int64, ctypes.c_int32, ctypes.c_float,
                                       ctypes.c_void_p]
+    lib.pe_geglu_fwd.restype = ctypes.c_int
+    lib.pe_geglu_fwd.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p]
     version = lib.pe_attn_abi_version()
     if version != ABI_VERSION:
         raise ImportError(f"{lib_path} has ABI {version}, expected {ABI_VERSION}: rebuild it")

@@ -618,4 +618,21 @@ int pe_layer_norm_fwd(const void *x, const void *residual, const void *weight, v
     return residual ? launch_norm<true>(p, stream) : launch_norm<false>(p, stream);
 }
 
+int pe_geglu_fwd(const void *proj, void *out, int64_t rows, int32_t width, hipStream_t stream) {
+    if (rows < 0 || width < 1) return PE_ATTN_EINVAL;
+    if (width & 7) return PE_ATTN_EUNSUPPORTED;
+    if (rows == 0) return PE_ATTN_OK;
+    if (!proj || !out || !aligned16(proj) || !aligned16(out)) return PE_ATTN_EINVAL;
+    pe::GegluParams p;
+    p.proj = static_cast<const __bf16 *>(proj);
+    p.out = static_cast<__bf16 *>(out);
+    p.per_row = width / 8;
+    if (rows > INT64_MAX / p.per_row) return PE_ATTN_EINVAL;
+    p.pieces = rows * p.per_row;
+    const int64_t blocks = p.pieces / 256 + (p.pieces % 256 != 0);
+    if (blocks > 0x7fffffffLL) return PE_ATTN_EUNSUPPORTED;
+    hipLaunchKernelGGL(pe::geglu_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, p);
+    return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
 }  // extern "C"

@@ -1,6 +1,7 @@
-// Row-wise passes of an encoder layer around its attention and products (gfx950): LayerNorm with
-// the residual add folded in, bound by HBM: every tensor is read or written once, in 16-byte
-// pieces, everything else stays in registers.
+// Elementwise and row-wise passes of an encoder layer around its attention and products (gfx950):
+// LayerNorm with the residual add folded in, and the GeGLU gate of the MLP. Both are bound by
+// HBM: every tensor is read or written once, in 16-byte pieces, everything else stays in
+// registers.
 #pragma once
 
 #include "pe_attn_device.h"
@@ -99,6 +100,57 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(NormParams p) {
         for (int j = 0; j < 8; ++j) y[j] = (__bf16)(((float)v[c][j] - mean) * rstd * (float)w[c][j]);
         if (i < pieces) *reinterpret_cast<bf16x8 *>(p.out + base + 8 * i) = y;
     }
+}
+
+// ----------------------------------------------------------------------------- GeGLU
+
+struct GegluParams {
+    const __bf16 *proj;  // [rows, 2 * width], contiguous: (input, gate)
+    __bf16 *out;         // [rows, width] (written)
+    int64_t pieces;      // rows * width / 8
+    int32_t per_row;     // width / 8
+};
+
+// gelu(x) = x * Phi(x), Phi the normal distribution function, written through its lower tail
+// Phi(-a) = t * 2^(Q(t) - a^2 log2(e) / 2), t = 1 / (1 + 0.22 a), a = |x|: the Gaussian factor is
+// taken out exactly and the rest is smooth in t, so one polynomial serves every a. Q is a degree-7
+// Chebyshev fit, on [0, 15], of log2(erfcx(a / sqrt 2) / 2) - log2(t); the fit's relative error is
+// 3.4e-7, also far out in the negative tail, where 1 + erf(x) loses its digits. Past 15 the power
+// of two underflows long before the polynomial matters. 18 VALU instructions and two transcendentals
+// per value, against about three times that for erff: with erff the pass is bound by the VALU, not
+// by memory.
+__device__ __forceinline__ float gelu(float x) {
+    const float a = __builtin_fabsf(x);
+    const float t = __builtin_amdgcn_rcpf(fmaf(0.22f, a, 1.0f));
+    float q = 0.601593779f;
+    q = fmaf(q, t, -2.31846865f);
+    q = fmaf(q, t, 3.11951201f);
+    q = fmaf(q, t, -2.07529329f);
+    q = fmaf(q, t, 1.29951664f);
+    q = fmaf(q, t, 0.409144346f);
+    q = fmaf(q, t, 1.47609864f);
+    q = fmaf(q, t, -3.51210317f);
+    const float tail = t * exp2_fast(fmaf(x * x, -0.5f * kLog2e, q));
+    return x * (x < 0.0f ? tail : 1.0f - tail);
+}
+
+// One thread per 16-byte output piece: gelu(input) * gate in fp32, rounded once. At 32,438 x 1,152:
+// 39.4 us for 224 MB (5.7 TB/s), against 70.6 + 38.9 us for torch's gelu and product, which also
+// write and read the rounded gelu.
+__global__ __launch_bounds__(256) void geglu_kernel(GegluParams p) {
+    const int64_t first = (int64_t)blockIdx.x * 256;  // the workgroup's first piece
+    const int64_t row0 = first / p.per_row;
+    const unsigned at = (unsigned)(first - row0 * p.per_row) + threadIdx.x;
+    if (first + threadIdx.x >= p.pieces) return;
+    const unsigned down = at / (unsigned)p.per_row;
+    const int64_t row = row0 + down;
+    const int64_t col = 8 * (int64_t)(at - down * (unsigned)p.per_row), width = 8 * (int64_t)p.per_row;
+    const __bf16 *src = p.proj + row * 2 * width + col;
+    const bf16x8 x = ld_g16(src), g = ld_g16(src + width);
+    bf16x8 y;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) y[j] = (__bf16)(gelu((float)x[j]) * (float)g[j]);
+    *reinterpret_cast<bf16x8 *>(p.out + row * width + col) = y;
 }
 
 }  // namespace pe

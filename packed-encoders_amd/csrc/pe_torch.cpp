@@ -102,9 +102,28 @@ PyObject *layer_norm(PyObject *, PyObject *const *args, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// geglu(proj) -> out, or None
+PyObject *geglu(PyObject *, PyObject *arg) {
+    HANDLE_TH_ERRORS
+    const Tensor *x = nullptr;
+    if (!plain_thread() || !plain_tensor(arg, x)) Py_RETURN_NONE;
+    const int64_t both = x->dim() ? x->size(-1) : 0;
+    if (both < 16 || both % 16 || both / 2 > INT32_MAX) Py_RETURN_NONE;
+    auto sizes = x->sizes().vec();
+    sizes.back() = both / 2;
+    Tensor out = at::empty(sizes, x->options());
+    if (failed(pe_geglu_fwd(x->const_data_ptr(), out.mutable_data_ptr(), x->numel() / both, (int32_t)(both / 2),
+                            stream_of(*x)),
+               "pe_geglu_fwd"))
+        return nullptr;
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
     {"layer_norm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(layer_norm)), METH_FASTCALL,
      "layer_norm(x, residual, weight, eps) -> out, (sum, out) or None"},
+    {"geglu", geglu, METH_O, "geglu(proj) -> out or None"},
     {nullptr, nullptr, 0, nullptr},
 };
 

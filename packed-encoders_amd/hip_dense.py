@@ -37,3 +37,7 @@ def layer_norm(x: Tensor, weight: Tensor, eps: float) -> Tensor | None:
 
 def add_layer_norm(x: Tensor, residual: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor] | None:
     return None if _off(x) or residual is None else _native().layer_norm(x, residual, weight, eps)
+
+
+def geglu(proj: Tensor) -> Tensor | None:
+    return None if _off(proj) else _native().geglu(proj)

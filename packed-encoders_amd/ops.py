@@ -8,7 +8,7 @@ fallback (ops.py:327-339), reached only when it is asked for.
 
 The rest of the layer has Hugging Face ModernBERT's numerics: LayerNorm without bias, bias-free
 linears, ``gelu(input) * gate``, split-half RoPE applied in fp32 with tables rounded to the model
-dtype. The linears are torch's; LayerNorm (with the residual add) and RoPE run on HIP kernels
+dtype. The linears are torch's; LayerNorm (with the residual add), GeGLU and RoPE run on HIP kernels
 for bf16 inference (``hip_dense``, ``hip_attention.rope_qkv``) and as plain torch ops otherwise.
 """
 
@@ -50,6 +50,9 @@ def dense_linear(x: Tensor, weight: Tensor) -> Tensor:
 
 def geglu(proj: Tensor) -> Tensor:
     """ModernBERT's MLP gate: the projection's halves ``(input, gate)`` → ``gelu(input) * gate``."""
+    out = hip_dense.geglu(proj)
+    if out is not None:
+        return out
     inp, gate = proj.chunk(2, dim=-1)
     return F.gelu(inp) * gate
 

@@ -1,4 +1,5 @@
-"""The LayerNorm kernel (with the residual add) against float64, and the calls it leaves to torch."""
+"""The LayerNorm (with the residual add) and GeGLU kernels against float64, and the calls they leave
+to torch."""
 
 from __future__ import annotations
 
@@ -54,6 +55,38 @@ def test_layer_norm_of_extreme_rows(pe):
     assert (out[0] == 0).all() and out[1].isnan().all() and out[2].isnan().all() and (out[3] == 0).all()
 
 
+def test_geglu_of_every_bf16_value(pe):
+    announce("geglu of every bf16 value")
+    bits = torch.arange(1 << 16, dtype=torch.int32, device="cuda").to(torch.int16)
+    x = bits.view(torch.bfloat16).view(-1, 64)
+    with torch.no_grad():
+        out = pe.ops.geglu(torch.cat((x, torch.ones_like(x)), -1))
+        torch_out = F.gelu(x)
+    want = F.gelu(x.double())
+    lower = x.double() * torch.special.erfc(x.double().abs() * 0.5 ** 0.5) * 0.5  # the negative tail's own digits
+    want = torch.where(x < 0, lower, want)
+    fine = x.isfinite()
+    err = (out.double() - want).abs()
+    # the output's rounding; the power of two's argument, up to 150, carries three fp32 roundings (150 * 3 *
+    # 2^-24 * ln 2 < 2^-15); Phi(x) under 2^-126 may be flushed to zero, |x| times that in the product
+    flushed = 2.0 ** -126 * x.double().abs().clamp(min=1)
+    assert (err[fine] <= ((HALF_STEP + 2.0 ** -15) * want.abs() + flushed)[fine]).all()
+    assert torch.equal(out[~fine].isnan(), torch_out[~fine].isnan())
+    assert torch.equal(out[x == float("inf")], x[x == float("inf")])
+
+
+@pytest.mark.parametrize("rows,width", [(1, 8), (7, 16), (3, 1152), (100, 1152), (31, 2624), (1000, 24)])
+def test_geglu_matches_float64(pe, rows, width):
+    announce(f"geglu {rows} x {width}")
+    proj = _bf16(2, rows, 2 * width, seed=width, std=2.0)
+    with torch.no_grad():
+        out = pe.ops.geglu(proj)
+    a, b = proj.double().chunk(2, -1)
+    want = F.gelu(a) * b
+    assert out.shape == want.shape
+    assert ((out.double() - want).abs() <= (HALF_STEP + 2.0 ** -15) * want.abs() + 1e-12).all()
+
+
 def test_other_calls_run_in_torch(pe):
     """Calls the kernels do not serve give torch's own results."""
     announce("dense calls left to torch")
@@ -61,15 +94,17 @@ def test_other_calls_run_in_torch(pe):
     for x in (_bf16(4, 768).float(), _bf16(4, 1536)[:, ::2], _bf16(4 * 768 + 1)[1:].view(4, 768), _bf16(4, 768).cpu()):
         ww = w.to(x.device, x.dtype)
         assert pe.hip_dense.layer_norm(x, ww, 1e-5) is None
-        assert pe.hip_dense.add_layer_norm(x, x, ww, 1e-5) is None
+        assert pe.hip_dense.add_layer_norm(x, x, ww, 1e-5) is None and pe.hip_dense.geglu(x) is None
         assert torch.equal(pe.ops.layer_norm(x, ww, 1e-5), F.layer_norm(x, (768,), ww, None, 1e-5))
+        assert torch.equal(pe.ops.geglu(x), F.gelu(x[..., :384]) * x[..., 384:])
     x = _bf16(4, 768)
-    assert pe.hip_dense.layer_norm(x[:, :12], w[:12], 1e-5) is None
+    assert pe.hip_dense.layer_norm(x[:, :12], w[:12], 1e-5) is None and pe.hip_dense.geglu(_bf16(4, 24)) is None
     with torch.autocast("cuda", dtype=torch.bfloat16):
         assert pe.ops.layer_norm(x, w, 1e-5).dtype == F.layer_norm(x, (768,), w, None, 1e-5).dtype
     x.requires_grad_()
-    pe.ops.add_layer_norm(x, x, w, 1e-5)[1].sum().backward()
+    pe.ops.geglu(pe.ops.add_layer_norm(x, x, w, 1e-5)[1]).sum().backward()
     assert x.grad is not None
     y = _bf16(3, 4, 768)
-    batched = torch.func.vmap(lambda t: pe.ops.layer_norm(t, w, 1e-5))(y)
-    assert torch.equal(batched, F.layer_norm(y, (768,), w, None, 1e-5))
+    batched = torch.func.vmap(lambda t: pe.ops.geglu(pe.ops.layer_norm(t, w, 1e-5)))(y)
+    each = torch.stack([F.gelu(n[:, :384]) * n[:, 384:] for n in F.layer_norm(y, (768,), w, None, 1e-5)])
+    assert torch.equal(batched, each)
