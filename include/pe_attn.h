@@ -138,6 +138,15 @@ const char *pe_attn_strerror(int status);
    device memory). */
 int pe_attn_workspace_size(const pe_attn_args *args, size_t *bytes);
 
+/* The chunks pe_varlen_attn_fwd cuts the longest key segment into when it spreads a call's key
+   segments over workgroups of their own (few query rows against long cu_seqlens_k segments), 1 when
+   it does not, or a negative status. A split call needs the whole pe_attn_workspace_size: the list
+   of pe_attn_plan and, behind it, the chunks' partial rows; with a workspace that holds the list
+   alone it runs unsplit, as the staged entry points always do (their workspace is only read by
+   pe_attn_tiled_fwd). A row read in several chunks agrees with the unsplit result within
+   rounding, one read in a single chunk bit for bit. Host-only. */
+int pe_attn_key_chunks(const pe_attn_args *args);
+
 /* Packed varlen attention, both kernels in one call. Segments are routed per segment on the
    device by their length (no host read of cu_seqlens): short ones to the LDS-resident kernel,
    long ones through a device-built, cost-ordered tile list to the tiled MFMA kernel.

@@ -360,6 +360,38 @@ int launch_tiled_d(const AttnParams &p, int g, bool gate, int64_t cap, hipStream
     return win ? launch_tiled_g<D, false, true>(p, g, cap, stream) : launch_tiled_g<D, false, false>(p, g, cap, stream);
 }
 
+// Split launches (pe_attn_split.h): one workgroup per work entry, head group and key chunk, then the
+// merge of every entry's rows.
+template <int D, int G>
+int launch_split_g(AttnParams p, int bm, int64_t cap, int chunks, hipStream_t stream) {
+    constexpr int BN = TiledShape<D>::BN, NS = TiledShape<D>::NS;
+    p.hgroups = p.hq / G;
+    const dim3 grid((unsigned)(cap * p.hgroups), chunks);
+    if constexpr (D == 64)
+        hipLaunchKernelGGL((pe::tiled_attn_kernel<D, G, BN, NS, false, true, true>), grid, dim3(256), 0, stream, p);
+    else if constexpr (D == 128)
+        hipLaunchKernelGGL((pe::wide_attn_kernel<D, G, BN, NS, false, true, true>), grid, dim3(256), 0, stream, p);
+    else
+        hipLaunchKernelGGL((pe::wide16_attn_kernel<D, kWide16Waves, G, NS, false, true, true>), grid,
+                           dim3(64 * kWide16Waves), 0, stream, p);
+    if (hipGetLastError() != hipSuccess) return PE_ATTN_ELAUNCH;
+    // rows of the longest tile the call can hold, in groups of 1024 / D
+    const int rows = p.max_seqlen < bm ? p.max_seqlen : bm;
+    const dim3 merge((unsigned)cap, p.hq, (rows * D + 1023) / 1024);
+    if (p.g)
+        hipLaunchKernelGGL((pe::merge_kernel<D, true>), merge, dim3(256), 0, stream, p, bm);
+    else
+        hipLaunchKernelGGL((pe::merge_kernel<D, false>), merge, dim3(256), 0, stream, p, bm);
+    return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
+template <int D>
+int launch_split_d(const AttnParams &p, int g, int bm, int64_t cap, int chunks, hipStream_t stream) {
+    if (g == 4) return launch_split_g<D, 4>(p, bm, cap, chunks, stream);
+    if (g == 2) return launch_split_g<D, 2>(p, bm, cap, chunks, stream);
+    return launch_split_g<D, 1>(p, bm, cap, chunks, stream);
+}
+
 int launch_tiled(const AttnParams &p, int d, int g, bool gate, int64_t cap, hipStream_t stream) {
     if (d == 64) return launch_tiled_d<64>(p, g, gate, cap, stream);
     if (d == 128) return launch_tiled_d<128>(p, g, gate, cap, stream);
@@ -390,11 +422,74 @@ int prepare(const pe_attn_args *a, Plan *plan) {
     return PE_ATTN_OK;
 }
 
+size_t list_bytes(int64_t cap) { return cap > 0 ? kWorkspaceHeader + (size_t)cap * sizeof(int4) : 0; }
+
+int64_t capacity_of(const pe_attn_args *a) {
+    return tile_capacity(a, effective_short_max(a), tile_rows(a, heads_per_tile(a)), effective_strip(a));
+}
+
+// A split of a call's key segments (pe_attn_split.h): the keys of a chunk, the most chunks a
+// segment has, and the bytes of their partial rows behind the list. No split: chunks 1, bytes 0.
+struct Split {
+    int chunk, chunks;
+    size_t offset, bytes;
+};
+
+// Splits calls with key segments of their own that would leave the chip waiting for a few long
+// walks, from host-known sizes. The chunk is the smallest (256 to 1,536 keys, in whole key tiles)
+// at which the call's workgroups still fit the chip at once: smaller chunks add partial rows and
+// rounds of short-lived workgroups, larger ones leave it idle. A call whose unsplit workgroups fill
+// the chip stays unsplit, as does one whose longest walk is at most 1,536 keys or barely more
+// than a chunk (the merge and the partial rows cost about 10 us). Measured, us, unsplit / chunk 256 /
+// 512 / 768 / 1,024 / 1,536, causal, by segments x keys, tails, heads x head_dim (the rule's choice):
+//   1 x 8,192, 1 row, 32:8 x 128                207 / 25 / 28 / 34 / 38 / 53        (256)
+//   4 x 4,096, 16 rows, 32:8 x 128              114 / 32 / 32 / 38 / 41 / 52        (320)
+//   16 x U{512..8192}, U{1..32}, 32:8 x 128     259 / 127 / 105 / 99 / 105 / 93     (1,408)
+//   64 x U{512..4096}, U{1..32}, 32:8 x 128     168 / 225 / 190 / 187 / 178 / 166   (1,536)
+//   24 x U{600..2000}, U{1..16}, 32:8 x 128     76 / 56 / 51 / 46 / 45 / 55         (640)
+//   64 x U{512..8192}, U{1..16}, 8:2 x 256      381 / 160 / 141 / 135 / 147 / 130   (1,280)
+//   16 x U{512..8192}, U{1..32}, 12:12 x 64     138 / 70 / 67 / 67 / 69 / 68        (1,408)
+constexpr int64_t kSplitMinChunk = 256, kSplitMaxChunk = 1536;
+constexpr size_t kSplitMaxBytes = (size_t)256 << 20;
+
+Split split_of(const pe_attn_args *a, int g, int bm, int64_t cap) {
+    Split s = {0, 1, 0, 0};
+    if (!a->cu_seqlens_k || cap == 0 || a->strip > 1 || a->total_tokens == 0 || global64(a)) return s;
+    // the most keys a query tile reads
+    const int wr = a->causal ? 0 : a->window_right;
+    int64_t reach = a->max_seqlen_k;
+    if (a->window_left >= 0 && wr >= 0 && (int64_t)bm + a->window_left + wr < reach) reach = (int64_t)bm + a->window_left + wr;
+    const int64_t slots = a->head_dim == 64 ? 3 * kCUs : 2 * kCUs;  // resident workgroups
+    const int64_t groups = cap * (a->n_heads_q / g);
+    if (reach <= kSplitMaxChunk || groups > slots) return s;
+    // A segment's chunks are its keys over the chunk and half a chunk more, on average; an eighth of
+    // the chip is left for uneven lengths (a few workgroups too many cost a whole round).
+    const int64_t keys = (int64_t)a->total_tokens_k / a->n_seq + 1, room = slots * 7 / 4 - groups;
+    int64_t chunk = (2 * groups * keys + room - 1) / room;
+    chunk = chunk < kSplitMinChunk ? kSplitMinChunk : chunk > kSplitMaxChunk ? kSplitMaxChunk : (chunk + 63) / 64 * 64;
+    if (2 * reach < 3 * chunk) return s;
+    const int chunks = (int)((a->max_seqlen_k + chunk - 1) / chunk);
+    const size_t rows = (size_t)chunks * a->total_tokens * a->n_heads_q;
+    if (chunks > 65535 || a->n_heads_q > 65535 || rows > kSplitMaxBytes / (4 * (a->head_dim + 2))) return s;
+    s.chunk = (int)chunk;
+    s.chunks = chunks;
+    s.offset = (list_bytes(cap) + 255) / 256 * 256;
+    s.bytes = rows * 4 * (a->head_dim + 2);
+    return s;
+}
+
 int check_workspace(const Plan &plan, const void *workspace, size_t bytes) {
-    if (plan.cap > 0 && (!workspace || !aligned16(workspace) ||
-                         bytes < kWorkspaceHeader + (size_t)plan.cap * sizeof(int4)))
+    if (plan.cap > 0 && (!workspace || !aligned16(workspace) || bytes < list_bytes(plan.cap)))
         return PE_ATTN_EWORKSPACE;
     return PE_ATTN_OK;
+}
+
+AttnParams planned_params(const pe_attn_args *a, const Plan &plan, const void *workspace) {
+    AttnParams p = make_params(a, plan.sm);
+    p.work_count = static_cast<const int32_t *>(workspace);
+    p.work = reinterpret_cast<const int4 *>(static_cast<const char *>(workspace) + kWorkspaceHeader);
+    p.work_cap = (int)plan.cap;
+    return p;
 }
 
 template <int D>
@@ -445,11 +540,18 @@ int pe_attn_workspace_size(const pe_attn_args *a, size_t *bytes) {
     if (!bytes) return PE_ATTN_EINVAL;
     const int rc = check_args(a, false);
     if (rc) return rc;
-    const int sm = effective_short_max(a);
+    const int64_t cap = capacity_of(a);
     const int g = heads_per_tile(a);
-    const int64_t cap = tile_capacity(a, sm, tile_rows(a, g), effective_strip(a));
-    *bytes = cap > 0 ? kWorkspaceHeader + (size_t)cap * sizeof(int4) : 0;
+    const Split split = split_of(a, g, tile_rows(a, g), cap);
+    *bytes = split.bytes ? split.offset + split.bytes : list_bytes(cap);
     return PE_ATTN_OK;
+}
+
+int pe_attn_key_chunks(const pe_attn_args *a) {
+    const int rc = check_args(a, false);
+    if (rc) return rc;
+    const int g = heads_per_tile(a);
+    return split_of(a, g, tile_rows(a, g), capacity_of(a)).chunks;
 }
 
 int pe_attn_plan(const pe_attn_args *a, void *workspace, size_t workspace_bytes, hipStream_t stream) {
@@ -485,10 +587,7 @@ int pe_attn_tiled_fwd(const pe_attn_args *a, const void *workspace, size_t works
     if (plan.cap == 0) return PE_ATTN_OK;
     rc = check_workspace(plan, workspace, workspace_bytes);
     if (rc) return rc;
-    AttnParams p = make_params(a, plan.sm);
-    p.work_count = static_cast<const int32_t *>(workspace);
-    p.work = reinterpret_cast<const int4 *>(static_cast<const char *>(workspace) + kWorkspaceHeader);
-    p.work_cap = (int)plan.cap;
+    const AttnParams p = planned_params(a, plan, workspace);
     return launch_tiled(p, a->head_dim, plan.g, a->gate != nullptr, plan.cap, stream);
 }
 
@@ -500,13 +599,26 @@ int pe_varlen_attn_fwd(const pe_attn_args *a, void *workspace, size_t workspace_
     if (rc) return rc;
     if ((rc = pe_attn_short_fwd(a, stream))) return rc;
     if ((rc = pe_attn_plan(a, workspace, workspace_bytes, stream))) return rc;
-    return pe_attn_tiled_fwd(a, workspace, workspace_bytes, stream);
+    // Split where the workspace holds the partial rows; one sized for the list alone runs unsplit.
+    const Split split = split_of(a, plan.g, plan.bm, plan.cap);
+    if (!split.bytes || workspace_bytes < split.offset + split.bytes)
+        return pe_attn_tiled_fwd(a, workspace, workspace_bytes, stream);
+    AttnParams p = planned_params(a, plan, workspace);
+    p.part_o = reinterpret_cast<float *>(static_cast<char *>(workspace) + split.offset);
+    p.part_ml = p.part_o + split.bytes / 4 / (a->head_dim + 2) * a->head_dim;
+    p.chunk = split.chunk;
+    p.total_q = a->total_tokens;
+    if (a->head_dim == 64) return launch_split_d<64>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
+    if (a->head_dim == 128) return launch_split_d<128>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
+    return launch_split_d<256>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
 }
 
 int pe_varlen_attn_fwd_noalloc(const pe_attn_args *a, hipStream_t stream) {
     size_t need = 0;
     int rc = pe_attn_workspace_size(a, &need);
     if (rc) return rc;
+    // Where the partial rows of a split do not fit, the list alone: the call then runs unsplit.
+    if (need > PE_ATTN_STATIC_SCRATCH_BYTES) need = list_bytes(capacity_of(a));
     if (need > PE_ATTN_STATIC_SCRATCH_BYTES) return PE_ATTN_ESCRATCH;
     void *ws = nullptr;
     if (need > 0 && (rc = static_scratch(&ws))) return rc;

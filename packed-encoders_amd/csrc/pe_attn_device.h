@@ -49,9 +49,21 @@ struct AttnParams {
     const int4 *work;          // tiled kernels: (segment, first q-tile, query start, query rows)
     const int32_t *work_count; // tiled kernels: number of valid entries
     int32_t work_cap;          // entries the workspace holds
-    const __bf16 *rcos, *rsin; // short kernel's fused RoPE tables [rows, D] (NULL: none)
-    int64_t rst;               // table row stride, elements
-    int32_t rrows;             // table rows: packed row r takes row r % rrows
+    // The short kernel's fused RoPE and the split calls share these (no call is both; a larger
+    // struct costs wide_attn_kernel 24 VGPRs of address arithmetic).
+    union {
+        struct {
+            const __bf16 *rcos, *rsin; // fused RoPE tables [rows, D] (NULL: none)
+            int64_t rst;               // table row stride, elements
+            int32_t rrows;             // table rows: packed row r takes row r % rrows
+        };
+        // pe_attn_split.h: unnormalised outputs [chunks][total_q][hq][D] of the chunks of `chunk`
+        // keys, and their maxima and sums [..][2], fp32.
+        struct {
+            float *part_o, *part_ml;
+            int32_t chunk, total_q;
+        };
+    };
 };
 
 // A tiled kernel's work item: the plan's (segment, first query tile, query start, query rows)

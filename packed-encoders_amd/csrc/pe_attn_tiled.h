@@ -51,7 +51,7 @@
 // (longest-processing-time order).
 #pragma once
 
-#include "pe_attn_stage.h"
+#include "pe_attn_split.h"
 
 namespace pe {
 
@@ -66,7 +66,7 @@ constexpr int kXcdRun = 4;
 // WIN: the call has a window or causal bound. Without one (global attention) every window
 // test folds away at compile time, which also gives global and windowed launches distinct
 // kernel names in traces.
-template <int D, int G, int BN, int NS, bool GATE, bool WIN>
+template <int D, int G, int BN, int NS, bool GATE, bool WIN, bool SPLIT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void tiled_attn_kernel(AttnParams p) {
     static_assert(D == 64 && BN == 64 && NS == 3, "head_dim 64 kernel (wider heads: wide_attn_kernel, wide16_attn_kernel)");
     static_assert(D % 32 == 0 && BN % 32 == 0 && (4 % G) == 0 && NS >= 2, "tile shape");
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     // longest-first order across XCDs (whole contiguous eighths would give one XCD all the
     // costliest tiles). The launch rounds the grid up to whole rounds of runs.
     int item = blockIdx.x;
-    if (WIN && p.wl >= 0 && p.wr >= 0) {
+    if (WIN && !SPLIT && p.wl >= 0 && p.wr >= 0) {
         const int rh = kXcdRun * p.hgroups;
         const int j = (int)(blockIdx.x >> 3);
         item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
@@ -106,14 +106,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows
-    const int kstart = wi.kstart, Lk = wi.Lk;  // keys
+    // SPLIT: the segment's keys end with the workgroup's chunk of them.
+    const int kstart = wi.kstart, Lk = SPLIT ? min(wi.Lk, ((int)blockIdx.y + 1) * p.chunk) : wi.Lk;  // keys
     // A segment longer than the caller's max_seqlen breaks the contract the host sized the
     // 32-bit buffer offsets by: its rows are left unwritten rather than addressed.
-    if (L > p.max_seqlen || Lk > p.max_seqlen_k || Lk < 0) return;
-    const int off = Lk - L;  // key position of query row 0 (queries end-aligned to their keys)
+    if (L > p.max_seqlen || wi.Lk > p.max_seqlen_k || Lk < 0) return;
+    const int off = wi.Lk - L;  // key position of query row 0 (queries end-aligned to their keys)
     const int nq = (L + BM - 1) / BM;
     if (qt_first >= nq) return;
     const int qt_end = min(nq, qt_first + p.strip);
+    if constexpr (SPLIT) {
+        // A tile that reads none of the chunk has nothing to add (the merge skips it by the same test).
+        const int chunk0 = blockIdx.y * p.chunk, q0 = qt_first * BM + off, q1 = min(L, qt_first * BM + BM) + off;
+        if (max(chunk0, p.wl >= 0 ? q0 - p.wl : 0) >= (p.wr >= 0 ? min(Lk, q1 + p.wr) : Lk)) return;
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -137,6 +143,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     auto key_range = [&](int qt, int &klo, int &ntiles) {
         const int q0 = qt * BM + off, rows_end = min(L, qt * BM + BM) + off;
         klo = wl >= 0 ? max(0, q0 - wl) : 0;
+        if constexpr (SPLIT) klo = max(klo, (int)blockIdx.y * p.chunk);
         const int khi = wr >= 0 ? min(Lk, rows_end + wr) : Lk;
         ntiles = max(1, (khi - klo + BN - 1) / BN);
     };
@@ -427,7 +434,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
         const bool via_lds = qt + 1 == qt_end;
         if (wave_active) {
             const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-            if (via_lds) {
+            if constexpr (SPLIT) {
+                store_part(o, m, lt, kg, p, start + myrow, qh, myrow < L);
+            } else if (via_lds) {
                 // `stage` already points past the last step's stage; the one before that is free.
                 const int free_stage = stage == 0 ? NS - 2 : stage == 1 ? NS - 1 : stage - 2;
                 store_rows<D, GATE>(o, inv, lane, &ring[free_stage][0][0] + wave * 32 * D, o_rs, r0 * (int)p.o_st * 2,

@@ -27,7 +27,7 @@ __host__ __device__ inline int xcd_run(int hgroups) {
 // This kernel: two 64 KB workgroups per CU (head_dim 128).
 __host__ __device__ inline int wide_run(int hgroups) { return xcd_run<64>(hgroups); }
 
-template <int D, int G, int BN, int NS, bool GATE, bool WIN>
+template <int D, int G, int BN, int NS, bool GATE, bool WIN, bool SPLIT = false>
 __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     static_assert(D % 32 == 0 && BN % 32 == 0 && (4 % G) == 0 && NS >= 2, "tile shape");
     constexpr int WPH = 4 / G;       // waves per query head
@@ -52,21 +52,27 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     // XCD's L2 (dealt one item per XCD, every tile fetched them again from memory).
     const int rh = wide_run(p.hgroups);
     const int j = (int)(blockIdx.x >> 3);
-    const int item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
+    const int item = SPLIT ? (int)blockIdx.x : ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
     const int entry = item / p.hgroups;
     const int hg = item - entry * p.hgroups;
     const WorkItem wi = load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows
-    const int kstart = wi.kstart, Lk = wi.Lk;  // keys
+    // SPLIT: the segment's keys end with the workgroup's chunk of them.
+    const int kstart = wi.kstart, Lk = SPLIT ? min(wi.Lk, ((int)blockIdx.y + 1) * p.chunk) : wi.Lk;  // keys
     // A segment longer than the caller's max_seqlen breaks the contract the host sized the
     // 32-bit buffer offsets by: its rows are left unwritten rather than addressed.
-    if (L > p.max_seqlen || Lk > p.max_seqlen_k || Lk < 0) return;
-    const int off = Lk - L;  // key position of query row 0 (queries end-aligned to their keys)
+    if (L > p.max_seqlen || wi.Lk > p.max_seqlen_k || Lk < 0) return;
+    const int off = wi.Lk - L;  // key position of query row 0 (queries end-aligned to their keys)
     const int nq = (L + BM - 1) / BM;
     if (qt_first >= nq) return;
     const int qt_end = min(nq, qt_first + p.strip);
+    if constexpr (SPLIT) {
+        // A tile that reads none of the chunk has nothing to add (the merge skips it by the same test).
+        const int chunk0 = blockIdx.y * p.chunk, q0 = qt_first * BM + off, q1 = min(L, qt_first * BM + BM) + off;
+        if (max(chunk0, p.wl >= 0 ? q0 - p.wl : 0) >= (p.wr >= 0 ? min(Lk, q1 + p.wr) : Lk)) return;
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -90,6 +96,7 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     auto key_range = [&](int qt, int &klo, int &ntiles) {
         const int q0 = qt * BM + off, rows_end = min(L, qt * BM + BM) + off;  // key positions
         klo = wl >= 0 ? max(0, q0 - wl) : 0;
+        if constexpr (SPLIT) klo = max(klo, (int)blockIdx.y * p.chunk);
         const int khi = wr >= 0 ? min(Lk, rows_end + wr) : Lk;
         ntiles = max(1, (khi - klo + BN - 1) / BN);
     };
@@ -329,7 +336,8 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
                 const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
                 const int ooff = myrow * (int)p.o_st * 2;
                 const int goff = GATE ? myrow * (int)p.g_st * 2 : 0;
-                store_block<DB, GATE>(o, inv, kg, o_rs, ooff, g_rs, goff);
+                if constexpr (SPLIT) store_part(o, m, lt, kg, p, start + myrow, qh, myrow < L);
+                else store_block<DB, GATE>(o, inv, kg, o_rs, ooff, g_rs, goff);
             }
             reset();
             if (qt + 1 >= qt_end) break;

@@ -71,7 +71,7 @@ __host__ __device__ inline int wide16_run(int hgroups) {
     return xcd_run<32 * (kByLds < kByWaves ? kByLds : kByWaves)>(hgroups);
 }
 
-template <int D, int NW, int G, int NS, bool GATE, bool WIN>
+template <int D, int NW, int G, int NS, bool GATE, bool WIN, bool SPLIT = false>
 __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
     static_assert(D == 256 && (NW == 4 || NW == 8) && (4 % G) == 0 && NS >= 2, "head_dim 256, 4 or 8 waves");
     constexpr int WPH = NW / G;      // waves per query head
@@ -91,21 +91,27 @@ __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
     // wide16_run() items dealt to the XCDs in turn).
     const int rh = wide16_run<NW, NS>(p.hgroups);
     const int j = (int)(blockIdx.x >> 3);
-    const int item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
+    const int item = SPLIT ? (int)blockIdx.x : ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
     const int entry = item / p.hgroups;
     const int hg = item - entry * p.hgroups;
     const WorkItem wi = load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows
-    const int kstart = wi.kstart, Lk = wi.Lk;  // keys
+    // SPLIT: the segment's keys end with the workgroup's chunk of them.
+    const int kstart = wi.kstart, Lk = SPLIT ? min(wi.Lk, ((int)blockIdx.y + 1) * p.chunk) : wi.Lk;  // keys
     // A segment longer than the caller's max_seqlen breaks the contract the host sized the
     // 32-bit buffer offsets by: its rows are left unwritten rather than addressed.
-    if (L > p.max_seqlen || Lk > p.max_seqlen_k || Lk < 0) return;
-    const int off = Lk - L;  // key position of query row 0 (queries end-aligned to their keys)
+    if (L > p.max_seqlen || wi.Lk > p.max_seqlen_k || Lk < 0) return;
+    const int off = wi.Lk - L;  // key position of query row 0 (queries end-aligned to their keys)
     const int nq = (L + BM - 1) / BM;
     if (qt_first >= nq) return;
     const int qt_end = min(nq, qt_first + p.strip);
+    if constexpr (SPLIT) {
+        // A tile that reads none of the chunk has nothing to add (the merge skips it by the same test).
+        const int chunk0 = blockIdx.y * p.chunk, q0 = qt_first * BM + off, q1 = min(L, qt_first * BM + BM) + off;
+        if (max(chunk0, p.wl >= 0 ? q0 - p.wl : 0) >= (p.wr >= 0 ? min(Lk, q1 + p.wr) : Lk)) return;
+    }
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -128,6 +134,7 @@ __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
     auto key_range = [&](int qt, int &klo, int &ntiles) {
         const int q0 = qt * BM + off, rows_end = min(L, qt * BM + BM) + off;  // key positions
         klo = wl >= 0 ? max(0, q0 - wl) : 0;
+        if constexpr (SPLIT) klo = max(klo, (int)blockIdx.y * p.chunk);
         const int khi = wr >= 0 ? min(Lk, rows_end + wr) : Lk;
         ntiles = max(1, (khi - klo + BN - 1) / BN);
     };
@@ -337,7 +344,9 @@ __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
             float lt = (ls[0] + ls[1]) + (ls[2] + ls[3]);
             lt += __shfl_xor(lt, 16);
             lt += __shfl_xor(lt, 32);
-            if (wave_active) {
+            if (SPLIT && wave_active) {
+                store_part16(o, m, lt, g4, p, start + myrow, qh, myrow < L);
+            } else if (wave_active) {
                 // Lane (c16, g4) rounds its 4-dim chunks (16 db + 4 g4 ..), then for each pair of
                 // 16-dim blocks (2j, 2j + 1) swap16_pair regroups the four lanes of a row so that
                 // lane g4 holds dims 32 j + 8 g4 .. + 7, whose gate factors it loaded: 16

@@ -168,7 +168,9 @@ def _varlen_impl(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_seqlen
                  min_seqlen=min_seqlen, rope=rope)
     stream = torch.cuda.current_stream(q.device).cuda_stream
     plans = _PLANS.get()
-    if plans is None:
+    # A call that splits its key segments writes partial rows into its workspace, so it takes one of
+    # its own: a shared plan is only read, by calls on any stream.
+    if plans is None or (cu_seqlens_k is not None and lib.pe_attn_key_chunks(ctypes.byref(args)) > 1):
         size = ctypes.c_size_t(0)
         _lib.check(lib.pe_attn_workspace_size(ctypes.byref(args), ctypes.byref(size)), "pe_attn_workspace_size")
         workspace = torch.empty(size.value, dtype=torch.uint8, device=q.device) if size.value else None

@@ -1,0 +1,166 @@
+"""Calls whose key segments are split into chunks over workgroups of their own (few query rows against
+long ``cu_seqlens_k`` segments): parity with the oracle at every chunk edge, the unsplit kernels' bits
+where a row reads one chunk, and graph replay."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+# keys around the 256-key chunk and the 64- and 32-key tiles; tails of one row, a part of a tile, a
+# tile and a row, none, and a tail longer than its keys (its first rows reach no key)
+KEYS = [1537, 256, 255, 257, 1024, 2100, 64, 0, 1600, 300, 2]
+TAILS = [1, 5, 32, 33, 16, 17, 64, 3, 0, 70, 9]
+# (head_dim, query heads, kv heads, window, causal, gate)
+CASES = [
+    (64, 4, 4, (-1, -1), True, False),
+    (64, 8, 2, (-1, 3), False, True),
+    (64, 6, 3, (1700, -1), True, False),
+    (128, 8, 2, (-1, -1), True, True),
+    (128, 4, 2, (-1, -1), False, False),
+    (128, 5, 5, (900, 900), False, False),
+    (256, 8, 2, (-1, -1), True, True),
+    (256, 4, 2, (-1, -1), False, False),
+    (256, 3, 3, (1600, -1), True, False),
+]
+
+
+def _inputs(d, hq, hkv, gate, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def draw(t, h):
+        return torch.randn(t, h, d, generator=g, device="cuda").bfloat16()
+
+    q, k, v = draw(sum(TAILS), hq), draw(sum(KEYS), hkv), draw(sum(KEYS), hkv)
+    return q, k, v, draw(sum(TAILS), hq) if gate else None
+
+
+def _cu(lengths):
+    return torch.tensor([0, *np.cumsum(lengths).tolist()], dtype=torch.int32, device="cuda")
+
+
+def _call(pe, case, q, k, v, gate, out, bytes_):
+    """The call through the C entry point with a workspace of `bytes_(chunks, size)` bytes."""
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    d, _, _, window, causal, _ = case
+    lib, cu, cuk = _lib.library(), _cu(TAILS), _cu(KEYS)
+    a = _args(q, k, v, out, cu, max(TAILS), d ** -0.5, *window, causal, gate, -1, cu_k=cuk, max_seqlen_k=max(KEYS))
+    size = ctypes.c_size_t()
+    assert lib.pe_attn_workspace_size(ctypes.byref(a), ctypes.byref(size)) == 0
+    n = bytes_(lib.pe_attn_key_chunks(ctypes.byref(a)), size.value)
+    ws = torch.full((n,), 0xFF, dtype=torch.uint8, device="cuda")  # partial rows nobody wrote would be NaN
+    assert lib.pe_varlen_attn_fwd(ctypes.byref(a), ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("case", CASES, ids=str)
+def test_split_call_matches_the_oracle_and_the_unsplit_kernel(pe, case):
+    announce(f"split {case}")
+    d, hq, hkv, window, causal, gated = case
+    q, k, v, gate = _inputs(d, hq, hkv, gated, seed=d + hq)
+    chunks = []
+    split = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda c, n: chunks.append(c) or n)
+    assert chunks == [9]  # 2,100 keys in chunks of 256, the smallest
+    # a workspace for the list alone (at most one entry per 16-row tile of each segment)
+    plain = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda c, n: 256 + 16 * len(KEYS) * 5)
+    want = pe.runtime_attention.oracle_attention(q, k, v, TAILS, KEYS, causal, window)
+    if gate is not None:
+        want = want * torch.sigmoid(gate.double())
+    for got in (split, plain):
+        assert (got.double() - want).abs().max() <= 2e-2
+        cos = torch.nn.functional.cosine_similarity(got.double().flatten(1), want.flatten(1), dim=-1)
+        seen = want.abs().amax(dim=(1, 2)) > 0
+        assert cos[seen].min() >= 0.9999
+    at = 0
+    for tail, keys in zip(TAILS, KEYS):
+        if keys <= 256:
+            assert torch.equal(split[at:at + tail], plain[at:at + tail]), (tail, keys)
+        at += tail
+
+
+def test_small_reaches_and_full_chips_stay_unsplit(pe):
+    """The rule, from host sizes alone: a window that spans few keys, a call whose tiles fill the
+    chip, shared key segments, strips and unbounded head_dim 64 calls are not split."""
+    from packed_encoders_amd import _lib
+
+    lib = _lib.library()
+
+    def chunks(d=128, n=8, tail=16, keys=4096, hq=32, hkv=8, own=True, **kw):
+        a = _lib.AttnArgs()
+        a.struct_size, a.dtype = ctypes.sizeof(_lib.AttnArgs), 1
+        a.n_seq, a.total_tokens, a.max_seqlen = n, n * tail, tail
+        a.n_heads_q, a.n_heads_kv, a.head_dim, a.softmax_scale = hq, hkv, d, d ** -0.5
+        a.window_left, a.window_right, a.causal, a.short_max = -1, -1, 1, -1
+        if own:
+            a.cu_seqlens_k, a.total_tokens_k, a.max_seqlen_k = 8, n * keys, keys
+        for name, value in kw.items():
+            setattr(a, name, value)
+        return lib.pe_attn_key_chunks(ctypes.byref(a))
+
+    assert chunks() == 7 and chunks(n=1) == 16 and chunks(keys=1537, n=1) == 7 and chunks(n=64, tail=1) == 3
+    assert chunks(d=256, n=4) == 13 and chunks(n=64) == 3
+    assert chunks(keys=1536) == chunks(own=False) == chunks(n=65) == chunks(tail=65, n=32) == 1
+    assert chunks(keys=2200, n=64) == 1 and chunks(keys=2304, n=64) == 2
+    assert chunks(window_left=1000) == 1 and chunks(window_left=1600) == 7
+    assert chunks(strip=2) == 1 and chunks(d=64, causal=0) == 1 and chunks(d=64, n=1) == 16
+    assert chunks(head_dim=96) == -2
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_split_call_replays_in_a_graph(pe, d):
+    announce(f"split call in a graph, head_dim {d}")
+    q, k, v, _ = _inputs(d, 8, 2, False, seed=d)
+    cu, cuk = _cu(TAILS), _cu(KEYS)
+
+    def call():
+        return pe.varlen_attention(q, k, v, cu, max(TAILS), causal=True, cu_seqlens_k=cuk, max_seqlen_k=max(KEYS))
+
+    with torch.inference_mode():
+        want = [call()]
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = call()
+        for i in range(4):
+            if i % 2:
+                k.neg_()
+                want.append(call())
+                torch.cuda.synchronize()
+            out.fill_(7.0)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want[-1]), i
+
+
+def test_split_calls_on_two_streams_share_nothing(pe):
+    """Calls in one shared_plans scope on two streams at once give the bits of the calls alone."""
+    announce("split calls on two streams")
+    a, b = _inputs(128, 8, 2, False, seed=1), _inputs(128, 8, 2, False, seed=2)
+    cu, cuk = _cu(TAILS), _cu(KEYS)
+
+    def call(t):
+        return pe.varlen_attention(t[0], t[1], t[2], cu, max(TAILS), causal=True, cu_seqlens_k=cuk,
+                                   max_seqlen_k=max(KEYS))
+
+    with torch.inference_mode():
+        want = call(a), call(b)
+        streams = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        with pe.shared_plans():
+            got = ([], [])
+            for _ in range(6):
+                for stream, t, outs in zip(streams, (a, b), got):
+                    with torch.cuda.stream(stream):
+                        outs.append(call(t))
+            torch.cuda.synchronize()
+    for w, outs in zip(want, got):
+        assert all(torch.equal(w, o) for o in outs)
