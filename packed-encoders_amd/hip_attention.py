@@ -24,6 +24,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from ._native import native_for
 
 _BF16 = torch.bfloat16
 
@@ -129,11 +130,30 @@ def shared_plans(min_seqlen: int = 0):
         _PLANS.reset(token)
 
 
+# The part of the argument struct a plan depends on: the sizes, the window, the routing and the key
+# segments (with the softmax scale, which the layers of a forward share).
+_PLAN_FIELDS = slice(_lib.AttnArgs.n_seq.offset, _lib.AttnArgs.rope_cos.offset)
+
+
 def _plan_key(args: _lib.AttnArgs, cu: Tensor, cu_k: Tensor | None = None) -> tuple:
-    kv = (None,) if cu_k is None else (id(cu_k), cu_k.data_ptr(), args.total_tokens_k, args.max_seqlen_k)
-    return (id(cu), cu.data_ptr(), cu.numel(), args.total_tokens, args.max_seqlen, args.n_heads_q,
-            args.n_heads_kv, args.head_dim, args.window_left, args.window_right, args.causal, args.short_max,
-            args.strip, args.band_kernel, args.min_seqlen, *kv)
+    return (id(cu), args.cu_seqlens, None if cu_k is None else id(cu_k), bytes(args)[_PLAN_FIELDS])
+
+
+def _run_planned(lib, plans: dict, args: _lib.AttnArgs, cu: Tensor, cu_k: Tensor | None, stream: int) -> None:
+    """The call of `args` over its scope's plan, built on the first call that needs it."""
+    key = _plan_key(args, cu, cu_k)
+    entry = plans.get(key)
+    ref = ctypes.byref(args)
+    if entry is None:
+        size = ctypes.c_size_t(0)
+        _lib.check(lib.pe_attn_workspace_size(ref, ctypes.byref(size)), "pe_attn_workspace_size")
+        workspace = torch.empty(size.value, dtype=torch.uint8, device=cu.device) if size.value else None
+        ptr = workspace.data_ptr() if workspace is not None else None
+        _lib.check(lib.pe_attn_plan(ref, ptr, size.value, stream), "pe_attn_plan")
+        entry = plans[key] = ((cu, cu_k), workspace, ptr, size.value)
+    _, _, ptr, nbytes = entry
+    _lib.check(lib.pe_attn_short_fwd(ref, stream), "pe_attn_short_fwd")
+    _lib.check(lib.pe_attn_tiled_fwd(ref, ptr, nbytes, stream), "pe_attn_tiled_fwd")
 
 
 def _table_rows(t: Tensor) -> Tensor:
@@ -178,19 +198,7 @@ def _varlen_impl(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_seqlen
                                         size.value, stream)
         _lib.check(status, "pe_varlen_attn_fwd")
         return out
-    key = _plan_key(args, cu_seqlens, cu_seqlens_k)
-    entry = plans.get(key)
-    if entry is None:
-        size = ctypes.c_size_t(0)
-        _lib.check(lib.pe_attn_workspace_size(ctypes.byref(args), ctypes.byref(size)), "pe_attn_workspace_size")
-        workspace = torch.empty(size.value, dtype=torch.uint8, device=q.device) if size.value else None
-        ptr = workspace.data_ptr() if workspace is not None else None
-        _lib.check(lib.pe_attn_plan(ctypes.byref(args), ptr, size.value, stream), "pe_attn_plan")
-        entry = plans[key] = ((cu_seqlens, cu_seqlens_k), workspace, size.value)
-    _, workspace, nbytes = entry
-    ptr = workspace.data_ptr() if workspace is not None else None
-    _lib.check(lib.pe_attn_short_fwd(ctypes.byref(args), stream), "pe_attn_short_fwd")
-    _lib.check(lib.pe_attn_tiled_fwd(ctypes.byref(args), ptr, nbytes, stream), "pe_attn_tiled_fwd")
+    _run_planned(lib, plans, args, cu_seqlens, cu_seqlens_k, stream)
     return out
 
 
@@ -355,14 +363,53 @@ def varlen_attention(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor, max_se
             raise ValueError("the fused RoPE prologue takes shared key segments (no cu_seqlens_k)")
         if max_seqlen_k is None:
             raise ValueError("cu_seqlens_k needs max_seqlen_k")
+    cos, sin = rope if rope is not None else (None, None)
+    out = _launch("attention", (q, k, v, cu_seqlens, gate, cu_seqlens_k, cos, sin), cu_seqlens,
+                  (int(max_seqlen), int(window[0]), int(window[1]), bool(causal), int(short_max),
+                   0 if cu_seqlens_k is None else int(max_seqlen_k), int(band_kernel), min_seqlen, scale), cu_seqlens_k)
+    if out is not None:
+        return out
+    if cu_seqlens_k is not None:
         return torch.ops.pe_hip.varlen_attention_kv(q, k, v, cu_seqlens, cu_seqlens_k, int(max_seqlen),
                                                     int(max_seqlen_k), scale, int(window[0]), int(window[1]),
                                                     bool(causal), gate, int(short_max), int(band_kernel),
                                                     min_seqlen)
     return torch.ops.pe_hip.varlen_attention(q, k, v, cu_seqlens, int(max_seqlen), scale,
                                              int(window[0]), int(window[1]), bool(causal), gate,
-                                             int(short_max), int(band_kernel), min_seqlen,
-                                             *(rope if rope is not None else (None, None)))
+                                             int(short_max), int(band_kernel), min_seqlen, cos, sin)
+
+
+def _launch(name: str, inputs: tuple, cu: Tensor, options: tuple, cu_k: Tensor | None = None) -> Tensor | None:
+    """An attention call launched natively (``csrc/pe_torch.cpp``), or None for one that the torch
+    operators take. Inside a ``shared_plans`` scope the native code only checks and fills the
+    arguments, and the scope's plan is used; calls with key segments of their own, which may need a
+    workspace of their own there, go through the operators."""
+    native = native_for(inputs[0])
+    if native is None:
+        return None
+    plans = _PLANS.get()
+    if plans is None:
+        return getattr(native, name)(*inputs, *options, 0)
+    if cu_k is not None:
+        return None
+    args = _lib.AttnArgs()
+    filled = getattr(native, name)(*inputs, *options, ctypes.addressof(args))
+    if filled is None:
+        return None
+    out, stream = filled
+    _run_planned(_lib.library(), plans, args, cu, None, stream)
+    return out
+
+
+def attention_qkv(qkv: Tensor, h: int, d: int, cos: Tensor, sin: Tensor, cu_seqlens: Tensor, max_seqlen: int, *,
+                  window: tuple[int, int], softmax_scale: float) -> Tensor | None:
+    """RoPE and attention of a packed projection ``qkv [1, T, 3*h*d]`` whose segments the short kernel
+    serves whole, returned as ``[1, T, h*d]``: ``varlen_attention(rope=)`` on its three views, without
+    making them. None for a call that does not fit."""
+    max_seqlen = int(max_seqlen)
+    return _launch("attention_qkv", (qkv, h, d, cu_seqlens, cos, sin), cu_seqlens,
+                   (max_seqlen, int(window[0]), int(window[1]), False, -1, 0, 0, min(_FLOOR.get(), max_seqlen),
+                    float(softmax_scale)))
 
 
 def packed_short_attention_supported(q: Tensor, k: Tensor, v: Tensor, cu_seqlens: Tensor,
@@ -460,6 +507,9 @@ def rope_qkv(qkv: Tensor, h: int, d: int, cos: Tensor, sin: Tensor) -> tuple[Ten
     (packed_encoders/_kernels/rope.py:302-349); ``ValueError`` for bad shapes or dtypes."""
     if not qkv.is_cuda:
         raise ValueError("rope_qkv runs on the HIP device")
+    native = native_for(qkv)
+    if native is not None and (pair := native.rope(qkv, int(h), int(d), cos, sin)) is not None:
+        return pair
     q, k = torch.ops.pe_hip.rope_qkv(qkv, cos, sin, int(h), int(d))
     return q, k
 

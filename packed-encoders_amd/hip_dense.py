@@ -8,36 +8,21 @@ names and return None for a call the kernels do not serve (``csrc/pe_torch.cpp``
 
 from __future__ import annotations
 
-from functools import lru_cache
-
-import torch
 from torch import Tensor
 
-from ._build import LIBRARY
-
-
-@lru_cache(maxsize=1)
-def _native():
-    """The extension module, or None without a built library; ``ImportError`` for a library built
-    without its extension."""
-    if not LIBRARY.exists():
-        return None
-    from . import _pe_torch
-
-    return _pe_torch
-
-
-def _off(x: Tensor) -> bool:
-    return not x.is_cuda or torch.compiler.is_compiling() or _native() is None
+from ._native import native_for
 
 
 def layer_norm(x: Tensor, weight: Tensor, eps: float) -> Tensor | None:
-    return None if _off(x) else _native().layer_norm(x, None, weight, eps)
+    native = native_for(x)
+    return None if native is None else native.layer_norm(x, None, weight, eps)
 
 
 def add_layer_norm(x: Tensor, residual: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor] | None:
-    return None if _off(x) or residual is None else _native().layer_norm(x, residual, weight, eps)
+    native = native_for(x)
+    return None if native is None or residual is None else native.layer_norm(x, residual, weight, eps)
 
 
 def geglu(proj: Tensor) -> Tensor | None:
-    return None if _off(proj) else _native().geglu(proj)
+    native = native_for(proj)
+    return None if native is None else native.geglu(proj)

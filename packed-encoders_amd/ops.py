@@ -191,6 +191,12 @@ def flash_attention_qkv_bshd(qkv: Tensor, h: int, d: int, *, cos: Tensor, sin: T
         return attention_bshd(q, k, view[:, :, 2], window=window, scaling=scaling, cu_seqlens=cu_seqlens,
                               max_seqlen=max_seqlen, backend=backend)
     varlen_attention = _load_hip_attention()
+    if cu_seqlens is not None and not torch.is_grad_enabled():
+        from .hip_attention import attention_qkv
+
+        out = attention_qkv(qkv, h, d, cos, sin, cu_seqlens, max_seqlen, window=window, softmax_scale=scaling)
+        if out is not None:
+            return out
     floor = None  # packed: the enclosing shared_plans scope's host bound
     if cu_seqlens is None:
         cu_seqlens = torch.arange(0, (b + 1) * s, s, dtype=torch.int32, device=qkv.device)
