@@ -193,7 +193,8 @@ int pe_attn_tiled_fwd(const pe_attn_args *args, const void *workspace, size_t wo
 int pe_packed_short_attn_fwd(const pe_attn_args *args, hipStream_t stream);
 
 /* The short kernel's static launch choice for a max_seqlen (no runtime autotuning):
-   out[0] = query rows per wave (block_m), out[1] = key capacity held in LDS,
+   out[0] = query rows per wave (block_m), out[1] = key capacity held in LDS (a launch whose
+   segments are at most 96 tokens holds 96 of the 128; pe_attn_kernels reports launches),
    out[2] = heads per workgroup, out[3] = waves per workgroup.
    Replaces select_packed_short_attention_config
    (packed_encoders/_kernels/triton_packed_attention.py:29-42). */

@@ -249,10 +249,11 @@ void short_shape(int max_len, int d, int *sk, int *hpw) {
         *hpw = *sk == 32 ? 4 : (*sk == 64 ? 2 : 1);
 }
 
-// hpw never exceeds the shape's default (short_shape), the most heads whose K and V fit LDS.
+// hpw never exceeds the shape's default (short_shape), the most heads whose K and V fit LDS (and for
+// a capacity of 96, which short_launch_shape takes, that of 128).
 template <int D, int SK, bool GATE>
 int launch_short_h(const AttnParams &p, int hpw, hipStream_t stream) {
-    constexpr int kMax = (D == 64 ? 4 : 2) * 64 / SK;  // short_shape's hpw (4, 4, 2 / 4, 2, 1)
+    constexpr int kMax = (D == 64 ? 4 : 2) * 64 / SK;  // short_shape's hpw (4, 4, 2, 2 / 4, 2, 1, 1)
     if constexpr (kMax >= 4)
         if (hpw == 4) return launch_short_t<D, SK, 4, GATE>(p, stream);
     if constexpr (kMax >= 2)
@@ -264,6 +265,7 @@ template <int D, bool GATE>
 int launch_short_d(const AttnParams &p, int sk, int hpw, hipStream_t stream) {
     if (sk == 32) return launch_short_h<D, 32, GATE>(p, hpw, stream);
     if (sk == 64) return launch_short_h<D, 64, GATE>(p, hpw, stream);
+    if (sk == 96) return launch_short_h<D, 96, GATE>(p, hpw, stream);
     return launch_short_h<D, 128, GATE>(p, hpw, stream);
 }
 
@@ -278,10 +280,25 @@ int short_heads(int hpw, int64_t n_seq, int hq) {
     return hpw;
 }
 
+// The shape a call launches: short_shape's, with two refinements that buy workgroups per CU.
+//  * Segments of at most 96 tokens take a capacity of 96 instead of 128: 48 instead of 64 KB for two
+//    heads of 64, three workgroups instead of two. 1,223 x U{12..92}: 100 -> 89 us (fused RoPE, where
+//    the tables made it one workgroup of 96 KB, 200 -> 121 us); 1,000 x U{4..96} at 8 x 128:
+//    101 -> 90 us.
+//  * With fused RoPE a workgroup also holds its keys' table rows, so from capacity 64 on it takes
+//    half the heads: 4,096 x U{16..64}: 48 KB, three per CU, against 80 KB, two, 250 -> 235 us;
+//    2,048 x U{64..128}: 64 KB against 96 KB, 473 -> 322 us; 1,024 x U{8..64} at 8 x 128:
+//    116 -> 101 us. At capacity 32 the default stays (two heads instead of four: 93 -> 111 us).
+void short_launch_shape(int max_len, int d, bool rope, int64_t n_seq, int hq, int *sk, int *hpw) {
+    short_shape(max_len, d, sk, hpw);
+    if (*sk == 128 && max_len <= 96) *sk = 96;
+    if (rope && *sk >= 64 && *hpw > 1) *hpw /= 2;
+    *hpw = short_heads(*hpw, n_seq, hq);
+}
+
 int launch_short(const AttnParams &p, int d, bool gate, int short_max, hipStream_t stream) {
     int sk, hpw;
-    short_shape(short_max, d, &sk, &hpw);
-    hpw = short_heads(hpw, p.n_seq, p.hq);
+    short_launch_shape(short_max, d, p.rcos != nullptr, p.n_seq, p.hq, &sk, &hpw);
     if (d == 64) return gate ? launch_short_d<64, true>(p, sk, hpw, stream) : launch_short_d<64, false>(p, sk, hpw, stream);
     if (d == 128) return gate ? launch_short_d<128, true>(p, sk, hpw, stream) : launch_short_d<128, false>(p, sk, hpw, stream);
     return PE_ATTN_EUNSUPPORTED;
@@ -656,8 +673,8 @@ int pe_attn_kernels(const pe_attn_args *a, int32_t out[6]) {
     if (rc) return rc;
     if (!out) return PE_ATTN_EINVAL;
     const int sm = effective_short_max(a);
-    int sk = 0, hpw = 0;
-    if (sm > 0) short_shape(sm, a->head_dim, &sk, &hpw);
+    int sk = 0, heads = 0;
+    if (sm > 0) short_launch_shape(sm, a->head_dim, a->rope_cos != nullptr, a->n_seq, a->n_heads_q, &sk, &heads);
     const int g = heads_per_tile(a);
     const int32_t max_k = a->cu_seqlens_k ? a->max_seqlen_k : a->max_seqlen;
     const bool tiled = a->n_seq > 0 && a->total_tokens > 0 && (a->max_seqlen > sm || max_k > sm);
@@ -672,7 +689,6 @@ int pe_attn_kernels(const pe_attn_args *a, int32_t out[6]) {
     out[1] = kernel;
     out[2] = tiled ? effective_strip(a) : 0;
     out[3] = tiled ? tile_rows(a, g) : 0;
-    const int heads = sk ? short_heads(hpw, a->n_seq, a->n_heads_q) : 0;
     const int64_t groups = heads ? (int64_t)a->n_seq * ((a->n_heads_q + heads - 1) / heads) : 0;
     out[4] = heads;
     out[5] = (int32_t)(groups < 0x7fffffff ? groups : 0x7fffffff);

@@ -41,7 +41,7 @@ constexpr int short_waves_per_eu() {
 template <int D, int SK, int HPW, bool GATE, bool ROPE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(short_waves_per_eu<D, SK, HPW, ROPE>())))
 void short_attn_kernel(AttnParams p) {
-    static_assert(SK % 32 == 0 && SK <= 128 && (4 % HPW) == 0, "short tile shape");
+    static_assert(SK % 32 == 0 && SK <= 128 && (4 % HPW) == 0, "short tile shape");  // 32, 64, 96 or 128 keys
     constexpr int NB = SK / 32;
     constexpr int DC = D / 16;
     constexpr int DB = D / 32;
@@ -104,17 +104,20 @@ void short_attn_kernel(AttnParams p) {
         }
     }
     if constexpr (ROPE) {
-        // Table rows of keys 0..SK-1 (row (kstart + key) % rrows), unit for unit as the K tile;
-        // keys past the segment take void loads (zeros, no traffic).
+        // Table rows of keys 0..SK-1 (row (kstart + key) % rrows: one scalar remainder and, for
+        // tables that wrap inside the segment, one per key), unit for unit as the K tile; keys
+        // past the segment take void loads (zeros, no traffic).
         const uint32_t tbytes = (uint32_t)((int64_t)p.rrows * p.rst * 2);
         const __amdgpu_buffer_rsrc_t c_rs = make_rsrc(p.rcos, tbytes), s_rs = make_rsrc(p.rsin, tbytes);
         const uint32_t tab_base = uniform((int)lds_addr(&tab[0][0]));
+        const unsigned rrows = (unsigned)p.rrows, row0 = (unsigned)kstart % rrows;
 #pragma unroll
         for (int j = 0; j < UPT; ++j) {
             const int u = (j * 4 + wave) * 64 + lane;
             const int key = u / CPR, ch = (u % CPR) ^ swz<CPR>(key);
-            const int row = (int)(((int64_t)kstart + key) % p.rrows);
-            const int off = key < Lk ? row * (int)p.rst * 2 + ch * 16 : kVoidOffset;
+            unsigned row = row0 + key;
+            if (row >= rrows) row %= rrows;
+            const int off = key < Lk ? (int)row * (int)p.rst * 2 + ch * 16 : kVoidOffset;
             const uint32_t dst = (uint32_t)uniform((int)(tab_base + (uint32_t)((j * 4 + wave) * 1024)));
             dma16(dst, off, c_rs);
             dma16(dst + TILE * 2, off, s_rs);
