@@ -455,9 +455,10 @@ struct Split {
 // Splits calls with key segments of their own that would leave the chip waiting for a few long
 // walks, from host-known sizes. The chunk is the smallest (256 to 1,536 keys, in whole key tiles)
 // at which the call's workgroups still fit the chip at once: smaller chunks add partial rows and
-// rounds of short-lived workgroups, larger ones leave it idle. A call whose unsplit workgroups fill
-// the chip stays unsplit, as does one whose longest walk is at most 1,536 keys or barely more
-// than a chunk (the merge and the partial rows cost about 10 us). Measured, us, unsplit / chunk 256 /
+// rounds of short-lived workgroups, larger ones leave it idle. A call of more than two unsplit
+// workgroups per CU stays unsplit (62 x U{478..3374} at 12:12 x 64, 744 workgroups: 85 us, split 94;
+// at 500 the two meet), as does one whose longest walk is at most 1,536 keys or barely more than a
+// chunk (the merge and the partial rows cost about 10 us). Measured, us, unsplit / chunk 256 /
 // 512 / 768 / 1,024 / 1,536, causal, by segments x keys, tails, heads x head_dim (the rule's choice):
 //   1 x 8,192, 1 row, 32:8 x 128                207 / 25 / 28 / 34 / 38 / 53        (256)
 //   4 x 4,096, 16 rows, 32:8 x 128              114 / 32 / 32 / 38 / 41 / 52        (320)
@@ -478,7 +479,7 @@ Split split_of(const pe_attn_args *a, int g, int bm, int64_t cap) {
     if (a->window_left >= 0 && wr >= 0 && (int64_t)bm + a->window_left + wr < reach) reach = (int64_t)bm + a->window_left + wr;
     const int64_t slots = a->head_dim == 64 ? 3 * kCUs : 2 * kCUs;  // resident workgroups
     const int64_t groups = cap * (a->n_heads_q / g);
-    if (reach <= kSplitMaxChunk || groups > slots) return s;
+    if (reach <= kSplitMaxChunk || groups > 2 * kCUs) return s;
     // A segment's chunks are its keys over the chunk and half a chunk more, on average; an eighth of
     // the chip is left for uneven lengths (a few workgroups too many cost a whole round).
     const int64_t keys = (int64_t)a->total_tokens_k / a->n_seq + 1, room = slots * 7 / 4 - groups;
