@@ -409,6 +409,43 @@ int launch_split_d(const AttnParams &p, int g, int bm, int64_t cap, int chunks, 
     return launch_split_g<D, 1>(p, bm, cap, chunks, stream);
 }
 
+// Whether a call runs without a plan: a narrow two-sided window (full tiles cost about the same in any
+// order; at +-600 that no longer holds and the longest-first plan is as good) in the tiled kernel,
+// over at most kDirectSegments segments. The plan kernel takes 5 to 9 us of such a call, finding a
+// tile from cu_seqlens about what reading its work entry takes. Calls with and without the plan, us,
+// 12 heads, +-64: 64 documents of median 400 tokens (300 tiles) 63.4 -> 59.5, 8 documents 21.0 -> 13.0,
+// 1 x 3,000 20.7 -> 12.7, 256 x median 300 174.5 -> 163.4; 64 documents causal with 256 keys to the left
+// 65.1 -> 60.3. 16 x 8,192 at 16 heads (16,384 tiles x heads) 237.3 -> 240.6, so the largest calls keep
+// it. The staged entry points do too: layers share their plan.
+constexpr int kDirectWindow = 256;
+constexpr int64_t kDirectMaxTiles = 12288;
+bool plans_itself(const pe_attn_args *a) {
+    const int wr = a->causal ? 0 : a->window_right;
+    return a->head_dim == 64 && a->window_left >= 0 && wr >= 0 && !a->cu_seqlens_k && a->strip <= 1 &&
+           (int64_t)a->window_left + wr <= kDirectWindow && a->n_seq <= pe::kDirectSegments &&
+           query_tiles(a) <= kDirectMaxTiles && !uses_band64(a);
+}
+
+template <int G>
+int launch_direct_g(AttnParams p, bool gate, int64_t cap, hipStream_t stream) {
+    constexpr int BN = TiledShape<64>::BN, NS = TiledShape<64>::NS;
+    p.hgroups = p.hq / G;
+    const int64_t run = 8LL * pe::kXcdRun * p.hgroups, blocks = (cap * p.hgroups + run - 1) / run * run;
+    if (blocks > 0x7fffffffLL) return PE_ATTN_EUNSUPPORTED;
+    const dim3 grid((unsigned)blocks), block(256);
+    if (gate)
+        hipLaunchKernelGGL((pe::tiled_attn_kernel<64, G, BN, NS, true, true, false, true>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((pe::tiled_attn_kernel<64, G, BN, NS, false, true, false, true>), grid, block, 0, stream, p);
+    return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
+int launch_direct(const AttnParams &p, int g, bool gate, int64_t cap, hipStream_t stream) {
+    if (g == 4) return launch_direct_g<4>(p, gate, cap, stream);
+    if (g == 2) return launch_direct_g<2>(p, gate, cap, stream);
+    return launch_direct_g<1>(p, gate, cap, stream);
+}
+
 int launch_tiled(const AttnParams &p, int d, int g, bool gate, int64_t cap, hipStream_t stream) {
     if (d == 64) return launch_tiled_d<64>(p, g, gate, cap, stream);
     if (d == 128) return launch_tiled_d<128>(p, g, gate, cap, stream);
@@ -616,6 +653,8 @@ int pe_varlen_attn_fwd(const pe_attn_args *a, void *workspace, size_t workspace_
     rc = check_workspace(plan, workspace, workspace_bytes);
     if (rc) return rc;
     if ((rc = pe_attn_short_fwd(a, stream))) return rc;
+    if (plan.cap > 0 && plans_itself(a))
+        return launch_direct(make_params(a, plan.sm), plan.g, a->gate != nullptr, plan.cap, stream);
     if ((rc = pe_attn_plan(a, workspace, workspace_bytes, stream))) return rc;
     // Split where the workspace holds the partial rows; one sized for the list alone runs unsplit.
     const Split split = split_of(a, plan.g, plan.bm, plan.cap);

@@ -95,6 +95,66 @@ __device__ __forceinline__ WorkItem load_work(const AttnParams &p, int entry) {
     return it;
 }
 
+// Inclusive sum over the wave's lanes: within rows of 16 (row_shr 1, 2, 4, 8), then each row's last
+// lane into the next row (row_bcast 15) and lane 31 into the upper half (row_bcast 31).
+__device__ __forceinline__ int wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+
+// The work item `entry` of a call that was not planned, found by every wave from the segment
+// boundaries: first the segments' full query tiles of bm rows in batch order, then their partial
+// last tiles (the cheaper ones, so that the launch ends on them). Lane l takes segments 4 l .. 4 l + 3
+// (at most kDirectSegments), a scan over the lanes numbers their tiles. For calls whose full tiles
+// all cost about the same; the same segments take tiles as in the plan (longer than short_max,
+// within the caller's bounds; keys are the queries').
+constexpr int kDirectSegments = 256;
+
+__device__ __forceinline__ WorkItem find_work(const AttnParams &p, int entry, int bm) {
+    const int lane = threadIdx.x & 63;
+    int bound[5], full[4], part[4], n_full = 0, n_part = 0;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) bound[i] = p.cu[min(4 * lane + i, p.n_seq)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int L = bound[i + 1] - bound[i];
+        const bool mine = L > p.short_max && L > 0 && L <= p.max_seqlen;
+        full[i] = mine ? L / bm : 0;
+        part[i] = mine && full[i] * bm < L ? 1 : 0;
+        n_full += full[i];
+        n_part += part[i];
+    }
+    const int full_upto = wave_scan(n_full), part_upto = wave_scan(n_part);
+    const int all_full = __builtin_amdgcn_readlane(full_upto, 63);
+    WorkItem it;
+    it.valid = entry >= 0 && entry < all_full + __builtin_amdgcn_readlane(part_upto, 63);
+    const bool last = entry >= all_full;
+    // The entry's lane is the last whose tiles begin at or before it; every lane finds the segment
+    // and tile as if it were that one.
+    const int want = last ? entry - all_full : entry, begin = last ? part_upto - n_part : full_upto - n_full;
+    int tile = want - begin, seg = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        const int n = last ? part[i] : full[i];
+        const bool past = seg == i && tile >= n;
+        tile -= past ? n : 0;
+        seg += past ? 1 : 0;
+    }
+    const int at = seg == 0 ? bound[0] : seg == 1 ? bound[1] : seg == 2 ? bound[2] : bound[3];
+    const int end = seg == 0 ? bound[1] : seg == 1 ? bound[2] : seg == 2 ? bound[3] : bound[4];
+    const int who = 63 - __builtin_clzll(__builtin_amdgcn_ballot_w64(begin <= want) | 1);
+    it.seg = 4 * who + __builtin_amdgcn_readlane(seg, who);
+    it.start = it.kstart = __builtin_amdgcn_readlane(at, who);
+    it.L = it.Lk = __builtin_amdgcn_readlane(end, who) - it.start;
+    it.qt_first = last ? it.L / bm : __builtin_amdgcn_readlane(tile, who);
+    return it;
+}
+
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // Buffer resources. A raw buffer (stride 0) whose range ends at the last byte of a segment's

@@ -65,8 +65,8 @@ constexpr int kXcdRun = 4;
 
 // WIN: the call has a window or causal bound. Without one (global attention) every window
 // test folds away at compile time, which also gives global and windowed launches distinct
-// kernel names in traces.
-template <int D, int G, int BN, int NS, bool GATE, bool WIN, bool SPLIT = false>
+// kernel names in traces. DIRECT: the call has no plan and finds its work items itself (find_work).
+template <int D, int G, int BN, int NS, bool GATE, bool WIN, bool SPLIT = false, bool DIRECT = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void tiled_attn_kernel(AttnParams p) {
     static_assert(D == 64 && BN == 64 && NS == 3, "head_dim 64 kernel (wider heads: wide_attn_kernel, wide16_attn_kernel)");
     static_assert(D % 32 == 0 && BN % 32 == 0 && (4 % G) == 0 && NS >= 2, "tile shape");
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     }
     const int entry = item / p.hgroups;
     const int hg = item - entry * p.hgroups;
-    const WorkItem wi = load_work(p, entry);
+    const WorkItem wi = DIRECT ? find_work(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows
