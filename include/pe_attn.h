@@ -143,8 +143,9 @@ int pe_attn_workspace_size(const pe_attn_args *args, size_t *bytes);
    it does not, or a negative status. A split call needs the whole pe_attn_workspace_size: the list
    of pe_attn_plan and, behind it, the chunks' partial rows; with a workspace that holds the list
    alone it runs unsplit, as the staged entry points always do (their workspace is only read by
-   pe_attn_tiled_fwd). A row read in several chunks agrees with the unsplit result within
-   rounding, one read in a single chunk bit for bit. Host-only. */
+   pe_attn_tiled_fwd). A row read in several chunks agrees with the unsplit long-segment kernel
+   within rounding, one read in a single chunk bit for bit; with short_max -1 a split call's short
+   segments take that kernel too. Host-only. */
 int pe_attn_key_chunks(const pe_attn_args *args);
 
 /* Packed varlen attention, both kernels in one call. Segments are routed per segment on the

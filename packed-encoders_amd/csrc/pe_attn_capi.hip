@@ -379,27 +379,43 @@ int launch_tiled_d(const AttnParams &p, int g, bool gate, int64_t cap, hipStream
 
 // Split launches (pe_attn_split.h): one workgroup per work entry, head group and key chunk, then the
 // merge of every entry's rows.
-template <int D, int G>
-int launch_split_g(AttnParams p, int bm, int64_t cap, int chunks, hipStream_t stream) {
+template <int D, int G, bool DIRECT>
+int launch_split_t(AttnParams p, int bm, int64_t cap, int chunks, hipStream_t stream) {
     constexpr int BN = TiledShape<D>::BN, NS = TiledShape<D>::NS;
     p.hgroups = p.hq / G;
-    const dim3 grid((unsigned)(cap * p.hgroups), chunks);
+    // Workgroup i runs on XCD i % 8: one workgroup past a multiple of 8 per chunk spreads a segment's
+    // chunks over the XCDs, which hold unequal shares of the keys otherwise.
+    const int64_t items = cap * p.hgroups;
+    const dim3 grid((unsigned)(items + (9 - items % 8) % 8), chunks);
     if constexpr (D == 64)
-        hipLaunchKernelGGL((pe::tiled_attn_kernel<D, G, BN, NS, false, true, true>), grid, dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((pe::tiled_attn_kernel<D, G, BN, NS, false, true, true, DIRECT>), grid, dim3(256), 0, stream, p);
     else if constexpr (D == 128)
-        hipLaunchKernelGGL((pe::wide_attn_kernel<D, G, BN, NS, false, true, true>), grid, dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((pe::wide_attn_kernel<D, G, BN, NS, false, true, true, DIRECT>), grid, dim3(256), 0, stream, p);
     else
-        hipLaunchKernelGGL((pe::wide16_attn_kernel<D, kWide16Waves, G, NS, false, true, true>), grid,
+        hipLaunchKernelGGL((pe::wide16_attn_kernel<D, kWide16Waves, G, NS, false, true, true, DIRECT>), grid,
                            dim3(64 * kWide16Waves), 0, stream, p);
     if (hipGetLastError() != hipSuccess) return PE_ATTN_ELAUNCH;
     // rows of the longest tile the call can hold, in groups of 1024 / D
     const int rows = p.max_seqlen < bm ? p.max_seqlen : bm;
     const dim3 merge((unsigned)cap, p.hq, (rows * D + 1023) / 1024);
     if (p.g)
-        hipLaunchKernelGGL((pe::merge_kernel<D, true>), merge, dim3(256), 0, stream, p, bm);
+        hipLaunchKernelGGL((pe::merge_kernel<D, true, DIRECT>), merge, dim3(256), 0, stream, p, bm);
     else
-        hipLaunchKernelGGL((pe::merge_kernel<D, false>), merge, dim3(256), 0, stream, p, bm);
+        hipLaunchKernelGGL((pe::merge_kernel<D, false, DIRECT>), merge, dim3(256), 0, stream, p, bm);
     return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
+// Small split calls (chunks under kSplitDirectChunk keys: the chip is not full) take their work items
+// without a plan, which is 4 to 5 us of 20 to 50: 1 x 8,192 keys 24.6 -> 19.2 us, 24 x U{600..2000}
+// 47 -> 41. Larger ones gain more from the plan's order, longest segments first: 16 x U{512..8192}
+// 91 us planned, 100 in batch order.
+constexpr int kSplitDirectChunk = 1024;
+bool split_direct(const AttnParams &p) { return p.n_seq <= pe::kDirectSegments && p.chunk < kSplitDirectChunk; }
+
+template <int D, int G>
+int launch_split_g(const AttnParams &p, int bm, int64_t cap, int chunks, hipStream_t stream) {
+    return split_direct(p) ? launch_split_t<D, G, true>(p, bm, cap, chunks, stream)
+                           : launch_split_t<D, G, false>(p, bm, cap, chunks, stream);
 }
 
 template <int D>
@@ -497,6 +513,7 @@ struct Split {
 // at 500 the two meet), as does one whose longest walk is at most 1,536 keys or barely more than a
 // chunk (the merge and the partial rows cost about 10 us). Measured, us, unsplit / chunk 256 /
 // 512 / 768 / 1,024 / 1,536, causal, by segments x keys, tails, heads x head_dim (the rule's choice):
+// (with the short pass and a plan; both are spared below)
 //   1 x 8,192, 1 row, 32:8 x 128                207 / 25 / 28 / 34 / 38 / 53        (256)
 //   4 x 4,096, 16 rows, 32:8 x 128              114 / 32 / 32 / 38 / 41 / 52        (320)
 //   16 x U{512..8192}, U{1..32}, 32:8 x 128     259 / 127 / 105 / 99 / 105 / 93     (1,408)
@@ -571,6 +588,27 @@ int launch_norm(const pe::NormParams &p, hipStream_t stream) {
     else
         hipLaunchKernelGGL((pe::layer_norm_kernel<8, ADD>), grid, block, 0, stream, p);
     return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
+// A call split into key chunks. By default its short segments take the split kernel as well, which
+// serves any length: that spares the short pass, 4.7 us of a 92 us call that has none of them.
+int launch_split(const pe_attn_args *call, const Split &split, void *workspace, size_t workspace_bytes,
+                 hipStream_t stream) {
+    pe_attn_args a = *call;
+    if (a.short_max < 0) a.short_max = 0;
+    Plan plan;
+    int rc = prepare(&a, &plan);
+    if (rc) return rc;
+    AttnParams p = planned_params(&a, plan, workspace);
+    p.part_o = reinterpret_cast<float *>(static_cast<char *>(workspace) + split.offset);
+    p.part_ml = p.part_o + split.bytes / 4 / (a.head_dim + 2) * a.head_dim;
+    p.chunk = split.chunk;
+    p.total_q = a.total_tokens;
+    if ((rc = pe_attn_short_fwd(&a, stream))) return rc;
+    if (!split_direct(p) && (rc = pe_attn_plan(&a, workspace, workspace_bytes, stream))) return rc;
+    if (a.head_dim == 64) return launch_split_d<64>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
+    if (a.head_dim == 128) return launch_split_d<128>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
+    return launch_split_d<256>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
 }
 
 }  // namespace
@@ -652,22 +690,15 @@ int pe_varlen_attn_fwd(const pe_attn_args *a, void *workspace, size_t workspace_
     if (rc) return rc;
     rc = check_workspace(plan, workspace, workspace_bytes);
     if (rc) return rc;
+    // Split where the workspace holds the partial rows; one sized for the list alone runs unsplit.
+    const Split split = split_of(a, plan.g, plan.bm, plan.cap);
+    if (split.bytes && workspace_bytes >= split.offset + split.bytes)
+        return launch_split(a, split, workspace, workspace_bytes, stream);
     if ((rc = pe_attn_short_fwd(a, stream))) return rc;
     if (plan.cap > 0 && plans_itself(a))
         return launch_direct(make_params(a, plan.sm), plan.g, a->gate != nullptr, plan.cap, stream);
     if ((rc = pe_attn_plan(a, workspace, workspace_bytes, stream))) return rc;
-    // Split where the workspace holds the partial rows; one sized for the list alone runs unsplit.
-    const Split split = split_of(a, plan.g, plan.bm, plan.cap);
-    if (!split.bytes || workspace_bytes < split.offset + split.bytes)
-        return pe_attn_tiled_fwd(a, workspace, workspace_bytes, stream);
-    AttnParams p = planned_params(a, plan, workspace);
-    p.part_o = reinterpret_cast<float *>(static_cast<char *>(workspace) + split.offset);
-    p.part_ml = p.part_o + split.bytes / 4 / (a->head_dim + 2) * a->head_dim;
-    p.chunk = split.chunk;
-    p.total_q = a->total_tokens;
-    if (a->head_dim == 64) return launch_split_d<64>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
-    if (a->head_dim == 128) return launch_split_d<128>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
-    return launch_split_d<256>(p, plan.g, plan.bm, plan.cap, split.chunks, stream);
+    return pe_attn_tiled_fwd(a, workspace, workspace_bytes, stream);
 }
 
 int pe_varlen_attn_fwd_noalloc(const pe_attn_args *a, hipStream_t stream) {

@@ -112,18 +112,28 @@ __device__ __forceinline__ int wave_scan(int x) {
 // last tiles (the cheaper ones, so that the launch ends on them). Lane l takes segments 4 l .. 4 l + 3
 // (at most kDirectSegments), a scan over the lanes numbers their tiles. For calls whose full tiles
 // all cost about the same; the same segments take tiles as in the plan (longer than short_max,
-// within the caller's bounds; keys are the queries').
+// within the caller's bounds). KEYS: the key segments are the call's own (cuk).
 constexpr int kDirectSegments = 256;
 
+template <bool KEYS = false>
 __device__ __forceinline__ WorkItem find_work(const AttnParams &p, int entry, int bm) {
     const int lane = threadIdx.x & 63;
-    int bound[5], full[4], part[4], n_full = 0, n_part = 0;
+    int bound[5], kbound[KEYS ? 5 : 1], full[4], part[4], n_full = 0, n_part = 0;
 #pragma unroll
-    for (int i = 0; i < 5; ++i) bound[i] = p.cu[min(4 * lane + i, p.n_seq)];
+    for (int i = 0; i < 5; ++i) {
+        bound[i] = p.cu[min(4 * lane + i, p.n_seq)];
+        if constexpr (KEYS) kbound[i] = p.cuk[min(4 * lane + i, p.n_seq)];
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int L = bound[i + 1] - bound[i];
-        const bool mine = L > p.short_max && L > 0 && L <= p.max_seqlen;
+        bool mine = L > 0 && L <= p.max_seqlen;
+        if constexpr (KEYS) {
+            const int Lk = kbound[i + 1] - kbound[i];
+            mine = mine && Lk >= 0 && Lk <= p.max_seqlen_k && max(L, Lk) > p.short_max;
+        } else {
+            mine = mine && L > p.short_max;
+        }
         full[i] = mine ? L / bm : 0;
         part[i] = mine && full[i] * bm < L ? 1 : 0;
         n_full += full[i];
@@ -151,6 +161,12 @@ __device__ __forceinline__ WorkItem find_work(const AttnParams &p, int entry, in
     it.seg = 4 * who + __builtin_amdgcn_readlane(seg, who);
     it.start = it.kstart = __builtin_amdgcn_readlane(at, who);
     it.L = it.Lk = __builtin_amdgcn_readlane(end, who) - it.start;
+    if constexpr (KEYS) {
+        const int kat = seg == 0 ? kbound[0] : seg == 1 ? kbound[1] : seg == 2 ? kbound[2] : kbound[3];
+        const int kend = seg == 0 ? kbound[1] : seg == 1 ? kbound[2] : seg == 2 ? kbound[3] : kbound[4];
+        it.kstart = __builtin_amdgcn_readlane(kat, who);
+        it.Lk = __builtin_amdgcn_readlane(kend, who) - it.kstart;
+    }
     it.qt_first = last ? it.L / bm : __builtin_amdgcn_readlane(tile, who);
     return it;
 }

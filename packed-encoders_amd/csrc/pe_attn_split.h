@@ -61,10 +61,10 @@ __device__ __forceinline__ void store_part16(const f32x4 (&o)[DB], float m, floa
 // maximum, so the result does not depend on which workgroup finished first. Bound by latency: the
 // loops are unrolled so that several chunks' loads are in flight, and each row group has a
 // workgroup of its own.
-template <int D, bool GATE>
+template <int D, bool GATE, bool DIRECT>
 __global__ __launch_bounds__(256) void merge_kernel(AttnParams p, int bm) {
     constexpr int LPR = D / 4, RPP = 256 / LPR;  // lanes per row, rows per pass
-    const WorkItem wi = load_work(p, blockIdx.x);
+    const WorkItem wi = DIRECT ? find_work<true>(p, blockIdx.x, bm) : load_work(p, blockIdx.x);
     if (!wi.valid || wi.L > p.max_seqlen || wi.Lk > p.max_seqlen_k || wi.Lk < 0) return;
     const int first = wi.qt_first * bm, last = min(wi.L, first + bm);
     if (first >= last) return;

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     }
     const int entry = item / p.hgroups;
     const int hg = item - entry * p.hgroups;
-    const WorkItem wi = DIRECT ? find_work(p, entry, BM) : load_work(p, entry);
+    const WorkItem wi = DIRECT ? find_work<SPLIT>(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows

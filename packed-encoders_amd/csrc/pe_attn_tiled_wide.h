@@ -28,7 +28,7 @@ __host__ __device__ inline int xcd_run(int hgroups) {
 // This kernel: two 64 KB workgroups per CU (head_dim 128).
 __host__ __device__ inline int wide_run(int hgroups) { return xcd_run<64>(hgroups); }
 
-template <int D, int G, int BN, int NS, bool GATE, bool WIN, bool SPLIT = false>
+template <int D, int G, int BN, int NS, bool GATE, bool WIN, bool SPLIT = false, bool DIRECT = false>
 __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     static_assert(D % 32 == 0 && BN % 32 == 0 && (4 % G) == 0 && NS >= 2, "tile shape");
     constexpr int WPH = 4 / G;       // waves per query head
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     const int item = SPLIT ? (int)blockIdx.x : ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
     const int entry = item / p.hgroups;
     const int hg = item - entry * p.hgroups;
-    const WorkItem wi = load_work(p, entry);
+    const WorkItem wi = DIRECT ? find_work<SPLIT>(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows

@@ -71,7 +71,7 @@ __host__ __device__ inline int wide16_run(int hgroups) {
     return xcd_run<32 * (kByLds < kByWaves ? kByLds : kByWaves)>(hgroups);
 }
 
-template <int D, int NW, int G, int NS, bool GATE, bool WIN, bool SPLIT = false>
+template <int D, int NW, int G, int NS, bool GATE, bool WIN, bool SPLIT = false, bool DIRECT = false>
 __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
     static_assert(D == 256 && (NW == 4 || NW == 8) && (4 % G) == 0 && NS >= 2, "head_dim 256, 4 or 8 waves");
     constexpr int WPH = NW / G;      // waves per query head
@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
     const int item = SPLIT ? (int)blockIdx.x : ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
     const int entry = item / p.hgroups;
     const int hg = item - entry * p.hgroups;
-    const WorkItem wi = load_work(p, entry);
+    const WorkItem wi = DIRECT ? find_work<SPLIT>(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;
     const int start = wi.start, L = wi.L;      // query rows

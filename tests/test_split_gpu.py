@@ -46,14 +46,14 @@ def _cu(lengths):
     return torch.tensor([0, *np.cumsum(lengths).tolist()], dtype=torch.int32, device="cuda")
 
 
-def _call(pe, case, q, k, v, gate, out, bytes_):
+def _call(pe, case, q, k, v, gate, out, bytes_, short_max=-1):
     """The call through the C entry point with a workspace of `bytes_(chunks, size)` bytes."""
     from packed_encoders_amd import _lib
     from packed_encoders_amd.hip_attention import _args
 
     d, _, _, window, causal, _ = case
     lib, cu, cuk = _lib.library(), _cu(TAILS), _cu(KEYS)
-    a = _args(q, k, v, out, cu, max(TAILS), d ** -0.5, *window, causal, gate, -1, cu_k=cuk, max_seqlen_k=max(KEYS))
+    a = _args(q, k, v, out, cu, max(TAILS), d ** -0.5, *window, causal, gate, short_max, cu_k=cuk, max_seqlen_k=max(KEYS))
     size = ctypes.c_size_t()
     assert lib.pe_attn_workspace_size(ctypes.byref(a), ctypes.byref(size)) == 0
     n = bytes_(lib.pe_attn_key_chunks(ctypes.byref(a)), size.value)
@@ -71,12 +71,14 @@ def test_split_call_matches_the_oracle_and_the_unsplit_kernel(pe, case):
     chunks = []
     split = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda c, n: chunks.append(c) or n)
     assert chunks == [9]  # 2,100 keys in chunks of 256, the smallest
-    # a workspace for the list alone (at most one entry per 16-row tile of each segment)
-    plain = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda c, n: 256 + 16 * len(KEYS) * 5)
+    # a workspace for the list alone (at most one entry per 16-row tile of each segment); a split call
+    # routes nothing to the short kernel by default
+    plain = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda c, n: 256 + 16 * len(KEYS) * 5, 0)
+    routed = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda c, n: n, 32 if d <= 128 else 0)
     want = pe.runtime_attention.oracle_attention(q, k, v, TAILS, KEYS, causal, window)
     if gate is not None:
         want = want * torch.sigmoid(gate.double())
-    for got in (split, plain):
+    for got in (split, plain, routed):
         assert (got.double() - want).abs().max() <= 2e-2
         cos = torch.nn.functional.cosine_similarity(got.double().flatten(1), want.flatten(1), dim=-1)
         seen = want.abs().amax(dim=(1, 2)) > 0
@@ -114,6 +116,21 @@ def test_small_reaches_and_full_chips_stay_unsplit(pe):
     assert chunks(window_left=1000) == 1 and chunks(window_left=1600) == 7
     assert chunks(strip=2) == 1 and chunks(d=64, causal=0) == 1 and chunks(d=64, n=1) == 16
     assert chunks(head_dim=96) == -2
+
+
+def test_split_call_of_many_segments_is_planned(pe):
+    """More segments than a wave numbers: the split kernel reads the plan's list."""
+    announce("split call of 300 segments")
+    rng = np.random.default_rng(3)
+    keys, tails = rng.integers(0, 40, size=300), rng.integers(0, 3, size=300)
+    keys[[0, 150, 299]], tails[[0, 150, 299]] = [1700, 2100, 1537], [2, 1, 2]
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(int(t), h, 128, generator=g, device="cuda").bfloat16()
+               for t, h in ((tails.sum(), 4), (keys.sum(), 1), (keys.sum(), 1)))
+    with torch.inference_mode():
+        got = pe.varlen_attention(q, k, v, _cu(tails), 2, causal=True, cu_seqlens_k=_cu(keys), max_seqlen_k=2100)
+    want = pe.runtime_attention.oracle_attention(q, k, v, tails, keys, True)
+    assert (got.double() - want).abs().max() <= 2e-2
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
