@@ -795,6 +795,26 @@ int pe_rope_qkv_fwd(const pe_rope_args *a, hipStream_t stream) {
     return launch_rope<256>(p, stream);
 }
 
+int pe_rope_rows_fwd(const int64_t *positions, float theta, int64_t rows, int32_t head_dim, void *cos, void *sin,
+                     hipStream_t stream) {
+    if (rows < 0 || !(theta > 0.0f)) return PE_ATTN_EINVAL;
+    if (head_dim != 64 && head_dim != 128 && head_dim != 256) return PE_ATTN_EUNSUPPORTED;
+    if (rows == 0) return PE_ATTN_OK;
+    if (!positions || !cos || !sin || !aligned16(cos) || !aligned16(sin)) return PE_ATTN_EINVAL;
+    if (rows > INT64_MAX / 16) return PE_ATTN_EINVAL;
+    const int64_t threads = rows * (head_dim / 16), blocks = threads / 256 + (threads % 256 != 0);
+    if (blocks > 0x7fffffffLL) return PE_ATTN_EUNSUPPORTED;
+    const pe::RopeRowsParams p = {positions, static_cast<__bf16 *>(cos), static_cast<__bf16 *>(sin), rows, theta};
+    const dim3 grid((unsigned)blocks), block(256);
+    if (head_dim == 64)
+        hipLaunchKernelGGL(pe::rope_rows_kernel<64>, grid, block, 0, stream, p);
+    else if (head_dim == 128)
+        hipLaunchKernelGGL(pe::rope_rows_kernel<128>, grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL(pe::rope_rows_kernel<256>, grid, block, 0, stream, p);
+    return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
+}
+
 int pe_layer_norm_fwd(const void *x, const void *residual, const void *weight, void *sum, void *out, int64_t rows,
                       int32_t cols, float eps, hipStream_t stream) {
     if (rows < 0 || cols < 1) return PE_ATTN_EINVAL;

@@ -334,21 +334,21 @@ def packed_forward(model: nn.Module, params: ModernBertParams, packed_ids: Tenso
 
 def packed_core(model: nn.Module, params: ModernBertParams, x: Tensor, cu_seqlens: Tensor, max_seqlen: int,
                 position_ids: Tensor, *, execution, min_seqlen: int = 0) -> Tensor:
-    """RoPE tables up to ``max_seqlen`` gathered per token, then ``core`` on ``[1, T, hidden]``
+    """RoPE tables per token (positions below ``max_seqlen``), then ``core`` on ``[1, T, hidden]``
     with the HIP backend. Shared by the eager packed forward and the graph runner's capture."""
     device, dtype, d = x.device, x.dtype, params.head_dim
-    cos_g, sin_g = execution.rope_tables(max_seqlen, d, params.global_rope_theta, device, dtype)
-    if params.local_rope_theta == params.global_rope_theta:
-        cos_l, sin_l = cos_g, sin_g
-    else:
-        cos_l, sin_l = execution.rope_tables(max_seqlen, d, params.local_rope_theta, device, dtype)
 
-    def gather(t: Tensor) -> Tensor:
-        return t[0].index_select(0, position_ids)[None]
+    def rows(theta: float) -> tuple[Tensor, Tensor]:
+        if execution.rope_tables is ops.rope_tables:
+            return ops.rope_rows(position_ids, max_seqlen, d, theta, dtype)
+        return tuple(t[0].index_select(0, position_ids)[None]
+                     for t in execution.rope_tables(max_seqlen, d, theta, device, dtype))
 
-    out = core(model, params, x[None], gather(cos_g), gather(sin_g), gather(cos_l), gather(sin_l), None, None,
-               execution=execution, backend="hip", cu_seqlens=cu_seqlens, max_seqlen=int(max_seqlen),
-               min_seqlen=min(int(min_seqlen), int(max_seqlen)))
+    cos_g, sin_g = rows(params.global_rope_theta)
+    same = params.local_rope_theta == params.global_rope_theta
+    cos_l, sin_l = (cos_g, sin_g) if same else rows(params.local_rope_theta)
+    out = core(model, params, x[None], cos_g, sin_g, cos_l, sin_l, None, None, execution=execution, backend="hip",
+               cu_seqlens=cu_seqlens, max_seqlen=int(max_seqlen), min_seqlen=min(int(min_seqlen), int(max_seqlen)))
     return out[0]
 
 

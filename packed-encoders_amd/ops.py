@@ -67,6 +67,20 @@ def rope_tables(seq_len: int, head_dim: int, theta: float, device, dtype) -> tup
     return emb.cos()[None].to(dtype), emb.sin()[None].to(dtype)
 
 
+def rope_rows(position_ids: Tensor, max_seqlen: int, head_dim: int, theta: float, dtype) -> tuple[Tensor, Tensor]:
+    """``rope_tables`` of each packed token's position, ``[1, T, head_dim]``: one HIP kernel for bf16
+    tables on the GPU, else the tables up to ``max_seqlen`` gathered by position."""
+    if dtype == torch.bfloat16:
+        from ._native import native_for
+
+        native = native_for(position_ids)
+        rows = None if native is None else native.rope_rows(position_ids, head_dim, theta)
+        if rows is not None:
+            return rows
+    cos, sin = rope_tables(max_seqlen, head_dim, theta, position_ids.device, dtype)
+    return cos[0].index_select(0, position_ids)[None], sin[0].index_select(0, position_ids)[None]
+
+
 def _rotate(x: Tensor, cos: Tensor, sin: Tensor) -> Tensor:
     xf = x.float()
     half = xf.shape[-1] // 2

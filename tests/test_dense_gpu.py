@@ -108,3 +108,15 @@ def test_other_calls_run_in_torch(pe):
     batched = torch.func.vmap(lambda t: pe.ops.geglu(pe.ops.layer_norm(t, w, 1e-5)))(y)
     each = torch.stack([F.gelu(n[:, :384]) * n[:, 384:] for n in F.layer_norm(y, (768,), w, None, 1e-5)])
     assert torch.equal(batched, each)
+
+
+@pytest.mark.parametrize("d,theta", [(64, 160000.0), (64, 10000.0), (128, 10000.0), (256, 500.0)])
+def test_rope_rows_are_the_gathered_tables(pe, d, theta):
+    announce(f"rope rows d={d} theta={theta}")
+    positions = torch.cat([torch.arange(n) for n in (1, 7, 8192, 300)]).cuda()
+    cos, sin = pe.ops.rope_rows(positions, 8192, d, theta, torch.bfloat16)
+    tables = pe.ops.rope_tables(8192, d, theta, torch.device("cuda"), torch.bfloat16)
+    for got, table in ((cos, tables[0]), (sin, tables[1])):
+        assert torch.equal(got, table[0].index_select(0, positions)[None])
+    half = pe.ops.rope_rows(positions, 8192, d, theta, torch.float32)[0]  # another type: the tables' path
+    assert half.dtype == torch.float32 and torch.equal(half.bfloat16(), cos)
