@@ -151,11 +151,11 @@ def kernel_instance(lib, call, workload):
         short = f"pe::short_attn_kernel<{d}, {out[0]}, {out[4]}, {gate}>"
     long = {
         _lib.KERNEL_NONE: None,
-        _lib.KERNEL_TILED: f"pe::tiled_attn_kernel<64, {g}, 64, 3, {gate}, {win}>",
+        _lib.KERNEL_TILED: f"pe::tiled_attn_kernel<64, {g}, 64, 3, {gate}, {win}, false, false>",
         _lib.KERNEL_GLOBAL64: f"pe::global64_attn_kernel<{g}, {gate}>",
         _lib.KERNEL_BAND64: f"pe::band64_attn_kernel<{gate}>",
-        _lib.KERNEL_WIDE: f"pe::wide_attn_kernel<128, {g}, 64, 2, {gate}, {win}>",
-        _lib.KERNEL_WIDE16: f"pe::wide16_attn_kernel<256, 4, {g}, 2, {gate}, {win}>",
+        _lib.KERNEL_WIDE: f"pe::wide_attn_kernel<128, {g}, 64, 2, {gate}, {win}, false, false>",
+        _lib.KERNEL_WIDE16: f"pe::wide16_attn_kernel<256, 4, {g}, 2, {gate}, {win}, false, false>",
     }[out[1]]
     return short, long
 
