@@ -246,11 +246,12 @@ int pe_rope_qkv_fwd(const pe_rope_args *args, hipStream_t stream);
 
 /* cos and sin [rows, head_dim] (bf16, contiguous, 16-byte aligned) of a packed batch's tokens: row r
    holds cos and sin of positions[r] * theta^(-2 i / head_dim), i < head_dim / 2, in both halves, in
-   fp32 rounded once: the per-token tables the RoPE entry points read. head_dim 64, 128 or 256.
+   fp32 rounded once: the per-token tables the RoPE entry points read. A position outside
+   [0, max_positions) has no row in the table this stands for: its rows are NaN. head_dim 64, 128 or 256.
    Replaces building the tables of every position and gathering them (packed_encoders/ops.py,
    forward.py:426-531). */
-int pe_rope_rows_fwd(const int64_t *positions, float theta, int64_t rows, int32_t head_dim, void *cos, void *sin,
-                     hipStream_t stream);
+int pe_rope_gather_fwd(const int64_t *positions, int64_t max_positions, float theta, int64_t rows, int32_t head_dim,
+                       void *cos, void *sin, hipStream_t stream);
 
 /* Bias-free LayerNorm of contiguous bf16 rows, with the residual add of an encoder layer folded
    in: s = bf16(x + residual) (or x when residual is NULL), out = bf16((s - mean(s)) *

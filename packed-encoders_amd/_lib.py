@@ -34,7 +34,7 @@ EXPORTED = (
     "pe_attn_short_config",
     "pe_attn_kernels",
     "pe_rope_qkv_fwd",
-    "pe_rope_rows_fwd",
+    "pe_rope_gather_fwd",
     "pe_layer_norm_fwd",
     "pe_geglu_fwd",
 )
@@ -144,9 +144,9 @@ def library(path: str | None = None) -> ctypes.CDLL:
     lib.pe_attn_kernels.argtypes = [ctypes.POINTER(AttnArgs), ctypes.POINTER(ctypes.c_int32)]
     lib.pe_rope_qkv_fwd.restype = ctypes.c_int
     lib.pe_rope_qkv_fwd.argtypes = [ctypes.POINTER(RopeArgs), ctypes.c_void_p]
-    lib.pe_rope_rows_fwd.restype = ctypes.c_int
-    lib.pe_rope_rows_fwd.argtypes = [ctypes.c_void_p, ctypes.c_float, ctypes.c_int64, ctypes.c_int32,
-                                     *[ctypes.c_void_p] * 3]
+    lib.pe_rope_gather_fwd.restype = ctypes.c_int
+    lib.pe_rope_gather_fwd.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_float, ctypes.c_int64,
+                                       ctypes.c_int32, *[ctypes.c_void_p] * 3]
     lib.pe_layer_norm_fwd.restype = ctypes.c_int
     lib.pe_layer_norm_fwd.argtypes = [*[ctypes.c_void_p] * 5, ctypes.c_int64, ctypes.c_int32, ctypes.c_float,
                                       ctypes.c_void_p]

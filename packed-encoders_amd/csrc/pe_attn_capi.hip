@@ -795,16 +795,17 @@ int pe_rope_qkv_fwd(const pe_rope_args *a, hipStream_t stream) {
     return launch_rope<256>(p, stream);
 }
 
-int pe_rope_rows_fwd(const int64_t *positions, float theta, int64_t rows, int32_t head_dim, void *cos, void *sin,
-                     hipStream_t stream) {
-    if (rows < 0 || !(theta > 0.0f)) return PE_ATTN_EINVAL;
+int pe_rope_gather_fwd(const int64_t *positions, int64_t max_positions, float theta, int64_t rows, int32_t head_dim,
+                       void *cos, void *sin, hipStream_t stream) {
+    if (rows < 0 || max_positions < 0 || !(theta > 0.0f)) return PE_ATTN_EINVAL;
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return PE_ATTN_EUNSUPPORTED;
     if (rows == 0) return PE_ATTN_OK;
     if (!positions || !cos || !sin || !aligned16(cos) || !aligned16(sin)) return PE_ATTN_EINVAL;
     if (rows > INT64_MAX / 16) return PE_ATTN_EINVAL;
     const int64_t threads = rows * (head_dim / 16), blocks = threads / 256 + (threads % 256 != 0);
     if (blocks > 0x7fffffffLL) return PE_ATTN_EUNSUPPORTED;
-    const pe::RopeRowsParams p = {positions, static_cast<__bf16 *>(cos), static_cast<__bf16 *>(sin), rows, theta};
+    const pe::RopeRowsParams p = {positions, static_cast<__bf16 *>(cos), static_cast<__bf16 *>(sin), rows, max_positions,
+                                  theta};
     const dim3 grid((unsigned)blocks), block(256);
     if (head_dim == 64)
         hipLaunchKernelGGL(pe::rope_rows_kernel<64>, grid, block, 0, stream, p);

@@ -56,13 +56,15 @@ struct RopeRowsParams {
     const int64_t *positions;  // [rows]
     __bf16 *cos, *sin;         // [rows, D], contiguous (written)
     int64_t rows;
+    int64_t max_positions;
     float theta;
 };
 
 // cos and sin rows of a packed batch's tokens: row r holds the angles positions[r] * theta^(-2 i / D) of
 // its position, each half of the row alike, in fp32 and rounded to bf16 (the arithmetic of building
-// the tables for every position and gathering them, in one launch instead of some fifteen). One
-// thread = 8 angles of a row, 16-byte stores.
+// the tables for every position and gathering them, in one launch instead of some fifteen). A
+// position outside [0, max_positions), which a gather could not read, gives NaN. One thread = 8
+// angles of a row, 16-byte stores.
 template <int D>
 __global__ __launch_bounds__(256) void rope_rows_kernel(RopeRowsParams p) {
     constexpr int CH = D / 16;  // 8-angle chunks per row
@@ -70,7 +72,8 @@ __global__ __launch_bounds__(256) void rope_rows_kernel(RopeRowsParams p) {
     const int64_t row = g / CH;
     if (row >= p.rows) return;
     const int c = (int)(g % CH);
-    const float pos = (float)p.positions[row];
+    const int64_t at = p.positions[row];
+    const float pos = (uint64_t)at < (uint64_t)p.max_positions ? (float)at : __builtin_nanf("");
     bf16x8 cs, sn;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {

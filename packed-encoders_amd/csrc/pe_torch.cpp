@@ -146,27 +146,28 @@ PyObject *geglu(PyObject *, PyObject *arg) {
     END_HANDLE_TH_ERRORS
 }
 
-// rope_rows(positions [T] int64, d, theta) -> (cos, sin) [1, T, d] bf16, or None
+// rope_rows(positions [T] int64, max_positions, d, theta) -> (cos, sin) [1, T, d] bf16, or None
 PyObject *rope_rows(PyObject *, PyObject *const *args, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    if (n != 3) {
-        PyErr_SetString(PyExc_TypeError, "rope_rows takes positions, d and theta");
+    if (n != 4) {
+        PyErr_SetString(PyExc_TypeError, "rope_rows takes positions, max_positions, d and theta");
         return nullptr;
     }
-    const int64_t d = PyLong_AsLongLong(args[1]);
-    if (d == -1 && PyErr_Occurred()) return nullptr;
-    const double theta = PyFloat_AsDouble(args[2]);
+    const int64_t max_positions = PyLong_AsLongLong(args[1]), d = PyLong_AsLongLong(args[2]);
+    if (PyErr_Occurred()) return nullptr;
+    const double theta = PyFloat_AsDouble(args[3]);
     if (theta == -1.0 && PyErr_Occurred()) return nullptr;
     const Tensor *pos = nullptr;
-    if ((d != 64 && d != 128 && d != 256) || !(theta > 0.0) || !plain_thread() ||
+    if (max_positions < 0 || (d != 64 && d != 128 && d != 256) || !(theta > 0.0) || !plain_thread() ||
         !plain_any(args[0], pos, at::kLong) || pos->dim() != 1 || !pos->is_contiguous() || pos->numel() == 0)
         Py_RETURN_NONE;
     const int64_t sizes[3] = {1, pos->numel(), d};
     const auto options = pos->options().dtype(at::kBFloat16);
     Tensor cos = at::empty(sizes, options), sin = at::empty(sizes, options);
-    if (failed(pe_rope_rows_fwd(static_cast<const int64_t *>(pos->const_data_ptr()), (float)theta, pos->numel(),
-                                (int32_t)d, cos.mutable_data_ptr(), sin.mutable_data_ptr(), stream_of(*pos)),
-               "pe_rope_rows_fwd"))
+    if (failed(pe_rope_gather_fwd(static_cast<const int64_t *>(pos->const_data_ptr()), max_positions, (float)theta,
+                                  pos->numel(), (int32_t)d, cos.mutable_data_ptr(), sin.mutable_data_ptr(),
+                                  stream_of(*pos)),
+               "pe_rope_gather_fwd"))
         return nullptr;
     PyObject *pair = PyTuple_New(2);
     if (!pair) return nullptr;
@@ -385,7 +386,7 @@ PyObject *attention_qkv(PyObject *, PyObject *const *args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"layer_norm", PE_FASTCALL(layer_norm), "layer_norm(x, residual, weight, eps) -> out, (sum, out) or None"},
     {"geglu", geglu, METH_O, "geglu(proj) -> out or None"},
-    {"rope_rows", PE_FASTCALL(rope_rows), "rope_rows(positions, d, theta) -> (cos, sin) or None"},
+    {"rope_rows", PE_FASTCALL(rope_rows), "rope_rows(positions, max_positions, d, theta) -> (cos, sin) or None"},
     {"rope", PE_FASTCALL(rope), "rope(qkv, h, d, cos, sin) -> (q, k) or None"},
     {"attention", PE_FASTCALL(attention),
      "attention(q, k, v, cu, gate, cu_k, cos, sin, max_seqlen, window_left, window_right, causal, short_max, "

@@ -69,12 +69,14 @@ def rope_tables(seq_len: int, head_dim: int, theta: float, device, dtype) -> tup
 
 def rope_rows(position_ids: Tensor, max_seqlen: int, head_dim: int, theta: float, dtype) -> tuple[Tensor, Tensor]:
     """``rope_tables`` of each packed token's position, ``[1, T, head_dim]``: one HIP kernel for bf16
-    tables on the GPU, else the tables up to ``max_seqlen`` gathered by position."""
+    tables on the GPU, else the tables up to ``max_seqlen`` gathered by position. Positions outside
+    ``[0, max_seqlen)`` have no row: the gather raises ``IndexError`` (a device assertion on the
+    GPU), the kernel, which cannot raise, gives NaN rows."""
     if dtype == torch.bfloat16:
         from ._native import native_for
 
         native = native_for(position_ids)
-        rows = None if native is None else native.rope_rows(position_ids, head_dim, theta)
+        rows = None if native is None else native.rope_rows(position_ids, int(max_seqlen), head_dim, theta)
         if rows is not None:
             return rows
     cos, sin = rope_tables(max_seqlen, head_dim, theta, position_ids.device, dtype)

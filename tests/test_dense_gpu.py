@@ -120,3 +120,17 @@ def test_rope_rows_are_the_gathered_tables(pe, d, theta):
         assert torch.equal(got, table[0].index_select(0, positions)[None])
     half = pe.ops.rope_rows(positions, 8192, d, theta, torch.float32)[0]  # another type: the tables' path
     assert half.dtype == torch.float32 and torch.equal(half.bfloat16(), cos)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_rope_rows_outside_the_table_are_nan(pe, d):
+    """Positions past ``max_seqlen`` or negative have no table row to gather: no angles come out for them."""
+    announce(f"rope rows outside the table d={d}")
+    positions = torch.tensor([0, 99, 100, 5, -1, 1 << 40, -(1 << 62), 42], device="cuda")
+    outside = torch.tensor([False, False, True, False, True, True, True, False], device="cuda")
+    for got, table in zip(pe.ops.rope_rows(positions, 100, d, 10000.0, torch.bfloat16),
+                          pe.ops.rope_tables(100, d, 10000.0, torch.device("cuda"), torch.bfloat16)):
+        assert torch.equal(got[0, ~outside], table[0].index_select(0, positions[~outside]))
+        assert got[0, outside].isnan().all()
+    with pytest.raises(IndexError):
+        pe.ops.rope_rows(positions.cpu(), 100, d, 10000.0, torch.bfloat16)
