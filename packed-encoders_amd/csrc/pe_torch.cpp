@@ -87,6 +87,21 @@ bool plain_tables(PyObject *cos_obj, PyObject *sin_obj, int64_t d, const Tensor 
 
 hipStream_t stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
+// Allocations and launches run without the interpreter lock: either can wait (a full queue, an
+// allocator that synchronises to free memory), and the process's other Python threads, host
+// callbacks among them, go on meanwhile. Everything they need is read from the tensors before; no
+// Python call is made inside.
+class Unlocked {
+  public:
+    Unlocked() : state_(PyEval_SaveThread()) {}
+    ~Unlocked() { PyEval_RestoreThread(state_); }
+    Unlocked(const Unlocked &) = delete;
+    Unlocked &operator=(const Unlocked &) = delete;
+
+  private:
+    PyThreadState *state_;
+};
+
 // The exception _lib.check raises for a status, or false for none.
 bool failed(int status, const char *what) {
     if (status == PE_ATTN_OK) return false;
@@ -112,13 +127,21 @@ PyObject *layer_norm(PyObject *, PyObject *const *args, Py_ssize_t n) {
         Py_RETURN_NONE;
     const double eps = PyFloat_AsDouble(args[3]);
     if (eps == -1.0 && PyErr_Occurred()) return nullptr;
-    Tensor out = at::empty(x->sizes(), x->options());
-    Tensor sum = add ? at::empty(x->sizes(), x->options()) : Tensor();
-    if (failed(pe_layer_norm_fwd(x->const_data_ptr(), add ? r->const_data_ptr() : nullptr, w->const_data_ptr(),
-                                 add ? sum.mutable_data_ptr() : nullptr, out.mutable_data_ptr(), x->numel() / cols,
-                                 (int32_t)cols, (float)eps, stream_of(*x)),
-               "pe_layer_norm_fwd"))
-        return nullptr;
+    const auto sizes = x->sizes().vec();
+    const auto options = x->options();
+    const void *src = x->const_data_ptr(), *res = add ? r->const_data_ptr() : nullptr, *weight = w->const_data_ptr();
+    const int64_t rows = x->numel() / cols;
+    const hipStream_t stream = stream_of(*x);
+    Tensor out, sum;
+    int status;
+    {
+        Unlocked unlocked;
+        out = at::empty(sizes, options);
+        if (add) sum = at::empty(sizes, options);
+        status = pe_layer_norm_fwd(src, res, weight, add ? sum.mutable_data_ptr() : nullptr, out.mutable_data_ptr(), rows,
+                                   (int32_t)cols, (float)eps, stream);
+    }
+    if (failed(status, "pe_layer_norm_fwd")) return nullptr;
     if (!add) return THPVariable_Wrap(std::move(out));
     PyObject *pair = PyTuple_New(2);
     if (!pair) return nullptr;
@@ -137,11 +160,18 @@ PyObject *geglu(PyObject *, PyObject *arg) {
     if (both < 16 || both % 16 || both / 2 > INT32_MAX) Py_RETURN_NONE;
     auto sizes = x->sizes().vec();
     sizes.back() = both / 2;
-    Tensor out = at::empty(sizes, x->options());
-    if (failed(pe_geglu_fwd(x->const_data_ptr(), out.mutable_data_ptr(), x->numel() / both, (int32_t)(both / 2),
-                            stream_of(*x)),
-               "pe_geglu_fwd"))
-        return nullptr;
+    const auto options = x->options();
+    const void *src = x->const_data_ptr();
+    const int64_t rows = x->numel() / both;
+    const hipStream_t stream = stream_of(*x);
+    Tensor out;
+    int status;
+    {
+        Unlocked unlocked;
+        out = at::empty(sizes, options);
+        status = pe_geglu_fwd(src, out.mutable_data_ptr(), rows, (int32_t)(both / 2), stream);
+    }
+    if (failed(status, "pe_geglu_fwd")) return nullptr;
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -163,12 +193,18 @@ PyObject *rope_rows(PyObject *, PyObject *const *args, Py_ssize_t n) {
         Py_RETURN_NONE;
     const int64_t sizes[3] = {1, pos->numel(), d};
     const auto options = pos->options().dtype(at::kBFloat16);
-    Tensor cos = at::empty(sizes, options), sin = at::empty(sizes, options);
-    if (failed(pe_rope_gather_fwd(static_cast<const int64_t *>(pos->const_data_ptr()), max_positions, (float)theta,
-                                  pos->numel(), (int32_t)d, cos.mutable_data_ptr(), sin.mutable_data_ptr(),
-                                  stream_of(*pos)),
-               "pe_rope_gather_fwd"))
-        return nullptr;
+    const int64_t *positions = static_cast<const int64_t *>(pos->const_data_ptr());
+    const hipStream_t stream = stream_of(*pos);
+    Tensor cos, sin;
+    int status;
+    {
+        Unlocked unlocked;
+        cos = at::empty(sizes, options);
+        sin = at::empty(sizes, options);
+        status = pe_rope_gather_fwd(positions, max_positions, (float)theta, sizes[1], (int32_t)d, cos.mutable_data_ptr(),
+                                    sin.mutable_data_ptr(), stream);
+    }
+    if (failed(status, "pe_rope_gather_fwd")) return nullptr;
     PyObject *pair = PyTuple_New(2);
     if (!pair) return nullptr;
     PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(std::move(cos)));
@@ -195,7 +231,8 @@ PyObject *rope(PyObject *, PyObject *const *args, Py_ssize_t n) {
     auto sizes = qkv->sizes().vec();
     sizes.back() = h;
     sizes.push_back(d);
-    Tensor q = at::empty(sizes, qkv->options()), k = at::empty(sizes, qkv->options());
+    const auto options = qkv->options();
+    const hipStream_t stream = stream_of(*qkv);
     pe_rope_args a;
     std::memset(&a, 0, sizeof(a));
     a.struct_size = sizeof(a);
@@ -203,15 +240,23 @@ PyObject *rope(PyObject *, PyObject *const *args, Py_ssize_t n) {
     a.qkv = qkv->const_data_ptr();
     a.cos = cos->const_data_ptr();
     a.sin = sin->const_data_ptr();
-    a.q_out = q.mutable_data_ptr();
-    a.k_out = k.mutable_data_ptr();
     a.qkv_stride_row = width;
     a.table_stride_row = d;
     a.table_rows = (int32_t)(cos->numel() / d);
     a.n_rows = (int32_t)(qkv->numel() / width);
     a.n_heads = (int32_t)h;
     a.head_dim = (int32_t)d;
-    if (failed(pe_rope_qkv_fwd(&a, stream_of(*qkv)), "pe_rope_qkv_fwd")) return nullptr;
+    Tensor q, k;
+    int status;
+    {
+        Unlocked unlocked;
+        q = at::empty(sizes, options);
+        k = at::empty(sizes, options);
+        a.q_out = q.mutable_data_ptr();
+        a.k_out = k.mutable_data_ptr();
+        status = pe_rope_qkv_fwd(&a, stream);
+    }
+    if (failed(status, "pe_rope_qkv_fwd")) return nullptr;
     PyObject *pair = PyTuple_New(2);
     if (!pair) return nullptr;
     PyTuple_SET_ITEM(pair, 0, THPVariable_Wrap(std::move(q)));
@@ -259,11 +304,27 @@ PyObject *finish(pe_attn_args &a, const Options &o, const Tensor &like, at::IntA
     a.short_max = (int32_t)o.short_max;
     a.band_kernel = (int32_t)o.band_kernel;
     a.min_seqlen = (int32_t)o.min_seqlen;
-    Tensor out = at::empty(sizes, like.options());
-    a.o = out.mutable_data_ptr();
     a.o_stride_head = a.head_dim;
     a.o_stride_token = (int64_t)a.n_heads_q * a.head_dim;
+    const auto shape = sizes.vec();
+    const auto options = like.options();
     const hipStream_t stream = stream_of(like);
+    Tensor out, workspace;
+    const char *what = "pe_attn_workspace_size";
+    int status = PE_ATTN_OK;
+    {
+        Unlocked unlocked;
+        out = at::empty(shape, options);
+        a.o = out.mutable_data_ptr();
+        size_t bytes = 0;
+        if (!o.args) status = pe_attn_workspace_size(&a, &bytes);
+        if (!o.args && status == PE_ATTN_OK) {
+            if (bytes) workspace = at::empty({(int64_t)bytes}, options.dtype(at::kByte));
+            what = "pe_varlen_attn_fwd";
+            status = pe_varlen_attn_fwd(&a, bytes ? workspace.mutable_data_ptr() : nullptr, bytes, stream);
+        }
+    }
+    if (failed(status, what)) return nullptr;
     if (o.args) {
         std::memcpy(o.args, &a, sizeof(a));
         PyObject *pair = PyTuple_New(2);
@@ -272,13 +333,6 @@ PyObject *finish(pe_attn_args &a, const Options &o, const Tensor &like, at::IntA
         PyTuple_SET_ITEM(pair, 1, PyLong_FromVoidPtr(stream));
         return pair;
     }
-    size_t bytes = 0;
-    if (failed(pe_attn_workspace_size(&a, &bytes), "pe_attn_workspace_size")) return nullptr;
-    Tensor workspace;
-    if (bytes) workspace = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
-    if (failed(pe_varlen_attn_fwd(&a, bytes ? workspace.mutable_data_ptr() : nullptr, bytes, stream),
-               "pe_varlen_attn_fwd"))
-        return nullptr;
     return THPVariable_Wrap(std::move(out));
 }
 

@@ -3,6 +3,11 @@ same bits on every form the native code takes, the operators' errors and copies 
 
 from __future__ import annotations
 
+import gc
+import sys
+import threading
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -115,3 +120,58 @@ def test_compiled_and_transformed_calls_see_the_operator(pe):
     with torch.no_grad(), Watch():
         got = pe.varlen_attention(q, q, q, cu, 30)
     assert torch.equal(got, want) and any("pe_hip" in name for name in seen)
+
+
+def _launches(pe):
+    """One call of every native launch, by name."""
+    h, d, T = 4, 64, 40
+    x, w = torch.randn(T, 512, device="cuda").bfloat16(), torch.ones(512, device="cuda").bfloat16()
+    qkv = torch.randn(1, T, 3 * h * d, device="cuda").bfloat16()
+    q, k, v = (qkv.view(T, 3, h, d)[:, i] for i in range(3))
+    positions, cu = torch.arange(T, device="cuda"), _cu([T])
+    cos, sin = (t[0] for t in pe.ops.rope_tables(T, d, 10000.0, torch.device("cuda"), torch.bfloat16))
+    return {
+        "layer_norm": lambda: pe.hip_dense.layer_norm(x, w, 1e-5),
+        "geglu": lambda: pe.hip_dense.geglu(x),
+        "rope_rows": lambda: pe.ops.rope_rows(positions, T, d, 10000.0, torch.bfloat16),
+        "rope": lambda: pe.hip_attention.rope_qkv(qkv, h, d, cos, sin),
+        "attention": lambda: pe.varlen_attention(q, k, v, cu, T),
+        "attention_qkv": lambda: pe.hip_attention.attention_qkv(qkv, h, d, cos, sin, cu, T, window=(-1, -1),
+                                                                softmax_scale=0.125),
+    }
+
+
+@pytest.mark.parametrize("name", ["layer_norm", "geglu", "rope_rows", "rope", "attention", "attention_qkv"])
+def test_other_threads_run_during_a_launch(pe, name):
+    """A launch or an allocation that has to wait must not stop the process's other Python threads: the
+    native calls give the interpreter lock up around both. With a switch interval that never passes,
+    another thread runs only where the calling one lets go by itself."""
+    announce(f"interpreter lock during {name}")
+    ran, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            ran[0] += 1
+            time.sleep(0)  # lets go and asks again
+
+    with torch.inference_mode():
+        call = _launches(pe)[name]
+        assert call() is not None
+        torch.cuda.synchronize()
+        thread = threading.Thread(target=other)
+        interval = sys.getswitchinterval()
+        sys.setswitchinterval(1000.0)
+        gc.disable()  # freeing a tensor lets go too: none is collected, the outputs are kept
+        try:
+            thread.start()
+            before, outs = ran[0], []
+            while ran[0] == before and len(outs) < 4000:
+                outs.append(call())
+            during = ran[0] - before
+        finally:
+            gc.enable()
+            sys.setswitchinterval(interval)
+            stop.set()
+            thread.join()
+        torch.cuda.synchronize()
+    assert during > 0
