@@ -23,7 +23,8 @@ def _module():
 
 def native_for(x: Tensor):
     """The extension module for a call on ``x``, or None where it has nothing to launch: tensors on
-    another device, calls that torch compiles, a package without its library."""
-    if not x.is_cuda or torch.compiler.is_compiling():
+    another device, calls that torch compiles, stand-ins that record a call (``torch.fx`` proxies), a
+    package without its library."""
+    if not isinstance(x, Tensor) or not x.is_cuda or torch.compiler.is_compiling():
         return None
     return _module()

@@ -1,0 +1,35 @@
+"""What the layer's functions do where no native launch is possible: recorded calls (CPU only)."""
+
+from __future__ import annotations
+
+import torch
+import torch.nn.functional as F
+
+
+def test_layer_functions_can_be_traced_symbolically(pe):
+    """``torch.fx`` records the norms and the gate: a proxy reaches the torch operations, and the
+    recorded graph gives their results."""
+    x, r, w = torch.randn(5, 32), torch.randn(5, 32), torch.randn(32)
+
+    class Layer(torch.nn.Module):
+        def forward(self, x, r, w):
+            s, n = pe.ops.add_layer_norm(x, r, w, 1e-5)
+            return s, pe.ops.geglu(n), pe.ops.layer_norm(x, w, 1e-5)
+
+    traced = torch.fx.symbolic_trace(Layer())
+    s, gated, n = traced(x, r, w)
+    a, b = F.layer_norm(x + r, (32,), w, None, 1e-5).chunk(2, -1)
+    assert torch.equal(s, x + r) and torch.equal(gated, F.gelu(a) * b)
+    assert torch.equal(n, F.layer_norm(x, (32,), w, None, 1e-5))
+
+
+def test_attention_calls_can_be_traced_symbolically(pe):
+    """A recorded attention call is the registered operator."""
+
+    class Layer(torch.nn.Module):
+        def forward(self, q, k, v, cu):
+            return pe.varlen_attention(q, k, v, cu, 64, window=(64, 64))
+
+    with torch.no_grad():
+        graph = torch.fx.symbolic_trace(Layer()).graph
+    assert any(node.target == torch.ops.pe_hip.varlen_attention for node in graph.nodes)
