@@ -27,15 +27,19 @@ BACKENDS = ("hip", "sdpa", "auto")
 
 
 def layer_norm(x: Tensor, weight: Tensor, eps: float) -> Tensor:
-    out = hip_dense.layer_norm(x, weight, eps)
-    return F.layer_norm(x, (x.shape[-1],), weight, None, eps) if out is None else out
+    if not torch.jit.is_scripting():  # a compiled script holds the torch operations alone
+        out = hip_dense.layer_norm(x, weight, eps)
+        if out is not None:
+            return out
+    return F.layer_norm(x, (x.shape[-1],), weight, None, eps)
 
 
 def add_layer_norm(x: Tensor, residual: Tensor, weight: Tensor, eps: float) -> tuple[Tensor, Tensor]:
     """``(x + residual, LayerNorm(x + residual))``: the residual stream and the next input."""
-    out = hip_dense.add_layer_norm(x, residual, weight, eps)
-    if out is not None:
-        return out
+    if not torch.jit.is_scripting():
+        out = hip_dense.add_layer_norm(x, residual, weight, eps)
+        if out is not None:
+            return out
     summed = x + residual
     return summed, layer_norm(summed, weight, eps)
 
@@ -50,9 +54,10 @@ def dense_linear(x: Tensor, weight: Tensor) -> Tensor:
 
 def geglu(proj: Tensor) -> Tensor:
     """ModernBERT's MLP gate: the projection's halves ``(input, gate)`` → ``gelu(input) * gate``."""
-    out = hip_dense.geglu(proj)
-    if out is not None:
-        return out
+    if not torch.jit.is_scripting():
+        out = hip_dense.geglu(proj)
+        if out is not None:
+            return out
     inp, gate = proj.chunk(2, dim=-1)
     return F.gelu(inp) * gate
 

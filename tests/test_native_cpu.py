@@ -33,3 +33,12 @@ def test_attention_calls_can_be_traced_symbolically(pe):
     with torch.no_grad():
         graph = torch.fx.symbolic_trace(Layer()).graph
     assert any(node.target == torch.ops.pe_hip.varlen_attention for node in graph.nodes)
+
+
+def test_layer_functions_compile_as_torchscript(pe):
+    x, r, w = torch.randn(5, 32), torch.randn(5, 32), torch.randn(32)
+    norm, add, gate = (torch.jit.script(f) for f in (pe.ops.layer_norm, pe.ops.add_layer_norm, pe.ops.geglu))
+    want = F.layer_norm(x + r, (32,), w, None, 1e-5)
+    s, n = add(x, r, w, 1e-5)
+    assert torch.equal(s, x + r) and torch.equal(n, want) and torch.equal(norm(x + r, w, 1e-5), want)
+    assert torch.equal(gate(x), F.gelu(x[:, :16]) * x[:, 16:])
