@@ -524,12 +524,20 @@ struct Split {
 constexpr int64_t kSplitMinChunk = 256, kSplitMaxChunk = 1536;
 constexpr size_t kSplitMaxBytes = (size_t)256 << 20;
 
+// A bound on the keys of one segment: max_seqlen_k or, where that is a capacity far above the lengths,
+// all the keys of the call. 16 x 1,000 keys, one row each, 32:8 x 128, max_seqlen_k 131,072: 342 chunks
+// of 384 keys for every segment took 97.6 us, 32 of 512 take 26.0, unsplit it is 42.7.
+int32_t longest_keys(const pe_attn_args *a) {
+    return a->max_seqlen_k < a->total_tokens_k ? a->max_seqlen_k : a->total_tokens_k;
+}
+
 Split split_of(const pe_attn_args *a, int g, int bm, int64_t cap) {
     Split s = {0, 1, 0, 0};
     if (!a->cu_seqlens_k || cap == 0 || a->strip > 1 || a->total_tokens == 0 || global64(a)) return s;
     // the most keys a query tile reads
     const int wr = a->causal ? 0 : a->window_right;
-    int64_t reach = a->max_seqlen_k;
+    const int64_t longest = longest_keys(a);
+    int64_t reach = longest;
     if (a->window_left >= 0 && wr >= 0 && (int64_t)bm + a->window_left + wr < reach) reach = (int64_t)bm + a->window_left + wr;
     const int64_t slots = a->head_dim == 64 ? 3 * kCUs : 2 * kCUs;  // resident workgroups
     const int64_t groups = cap * (a->n_heads_q / g);
@@ -538,9 +546,16 @@ Split split_of(const pe_attn_args *a, int g, int bm, int64_t cap) {
     // the chip is left for uneven lengths (a few workgroups too many cost a whole round).
     const int64_t keys = (int64_t)a->total_tokens_k / a->n_seq + 1, room = slots * 7 / 4 - groups;
     int64_t chunk = (2 * groups * keys + room - 1) / room;
+    // Every work entry launches a workgroup for each chunk the longest segment can have, and those past
+    // a segment's keys exit at once: eight rounds of the resident workgroups in all, at most. It matters
+    // where the bound is far above the lengths, us unsplit / chunk 256 / this rule, one row each,
+    // max_seqlen_k 8,192, head_dim 128: 32 x 300 keys, 32:8 heads, 26.6 / 30.6 (16 rounds) / 21.6;
+    // 200 x 200 keys, 8:2 heads, 27.1 / 34.0 (25) / 25.1. Four rounds cost 16 x 1,000 keys 26 -> 34.
+    const int64_t within = longest * groups / (8 * slots);
+    if (chunk < within) chunk = within;
     chunk = chunk < kSplitMinChunk ? kSplitMinChunk : chunk > kSplitMaxChunk ? kSplitMaxChunk : (chunk + 63) / 64 * 64;
     if (2 * reach < 3 * chunk) return s;
-    const int chunks = (int)((a->max_seqlen_k + chunk - 1) / chunk);
+    const int chunks = (int)((longest + chunk - 1) / chunk);
     const size_t rows = (size_t)chunks * a->total_tokens * a->n_heads_q;
     if (chunks > 65535 || a->n_heads_q > 65535 || rows > kSplitMaxBytes / (4 * (a->head_dim + 2))) return s;
     s.chunk = (int)chunk;
@@ -596,6 +611,7 @@ int launch_split(const pe_attn_args *call, const Split &split, void *workspace, 
                  hipStream_t stream) {
     pe_attn_args a = *call;
     if (a.short_max < 0) a.short_max = 0;
+    a.max_seqlen_k = longest_keys(&a);  // what the partial rows are sized for: a longer segment is skipped
     Plan plan;
     int rc = prepare(&a, &plan);
     if (rc) return rc;

@@ -181,3 +181,35 @@ def test_split_calls_on_two_streams_share_nothing(pe):
             torch.cuda.synchronize()
     for w, outs in zip(want, got):
         assert all(torch.equal(w, o) for o in outs)
+
+
+def _chunks(n, tail, keys, bound, hq=32, hkv=8, d=128):
+    from packed_encoders_amd import _lib
+
+    a = _lib.AttnArgs()
+    a.struct_size, a.dtype = ctypes.sizeof(_lib.AttnArgs), 1
+    a.n_seq, a.total_tokens, a.max_seqlen = n, n * tail, tail
+    a.n_heads_q, a.n_heads_kv, a.head_dim, a.softmax_scale = hq, hkv, d, d ** -0.5
+    a.window_left, a.window_right, a.causal, a.short_max = -1, -1, 1, -1
+    a.cu_seqlens_k, a.total_tokens_k, a.max_seqlen_k = 8, n * keys, bound
+    return _lib.library().pe_attn_key_chunks(ctypes.byref(a))
+
+
+def test_a_bound_far_above_the_lengths_adds_no_chunks(pe):
+    """max_seqlen_k may be a capacity: no segment holds more keys than the call, and the workgroups of
+    chunks that a segment does not have stay few."""
+    assert _chunks(1, 1, 500, 131072) == 1  # 500 keys in all: nothing to split
+    assert _chunks(16, 1, 1000, 131072) == _chunks(16, 1, 1000, 16000) <= 42
+    assert _chunks(32, 1, 300, 8192) * 32 * 8 <= 8 * 512 + 32 * 8  # eight rounds of two workgroups per CU
+    assert _chunks(1, 1, 8192, 131072) == _chunks(1, 1, 8192, 8192) == 32
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_split_call_under_a_loose_bound(pe, d):
+    announce(f"split call, max_seqlen_k a capacity, head_dim {d}")
+    q, k, v, _ = _inputs(d, 8, 2, False, seed=d)
+    with torch.inference_mode():
+        got = pe.varlen_attention(q, k, v, _cu(TAILS), max(TAILS), causal=True, cu_seqlens_k=_cu(KEYS),
+                                  max_seqlen_k=1 << 20)
+    want = pe.runtime_attention.oracle_attention(q, k, v, TAILS, KEYS, True)
+    assert (got.double() - want).abs().max() <= 2e-2
