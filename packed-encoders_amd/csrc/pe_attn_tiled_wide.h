@@ -1,11 +1,10 @@
 // Tiled packed attention for head_dim 128 (gfx950 MFMA; head_dim 256 runs the 16-row
 // wide16_attn_kernel, pe_attn_tiled_wide16.h, built on this one): the same workgroup shape,
-// LDS ring, direct global-to-LDS staging, swizzles and buffer-bounded accesses as
+// LDS ring, direct global-to-LDS staging, Q steps, swizzles and buffer-bounded accesses as
 // tiled_attn_kernel (pe_attn_tiled.h), with a step loop shaped for the register budget of
-// wide heads, whose O accumulators alone take D / 2 VGPRs per lane: the query rows loaded straight
-// into registers, one copy of the step (the ring stage is a register), the exact running maximum of
-// every tile (lazy rescale above 2^8), and loads issued only for real steps, the wait count
-// following how many are in flight. The
+// wide heads, whose O accumulators alone take D / 2 VGPRs per lane: one copy of the step (the
+// ring stage is a register), the exact running maximum of every tile (lazy rescale above 2^8),
+// and loads issued only for real steps, the wait count following how many are in flight. The
 // row sums add the bf16-rounded probabilities the P.V product uses (v_dot2 with ones), as the
 // head_dim 64 kernels do: under the lazily raised maximum a row's dominant probability is not
 // exactly 1, and summing it unrounded would leave its bf16 rounding (up to 2^-9 relative) in
@@ -40,7 +39,10 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     constexpr int TILE = BN * D;     // elements of one K (or V) tile
     constexpr int UPW = TILE / 8 / 64 / 4;  // 1 KB wave-loads per tensor per wave and tile
     constexpr int LPS = 2 * UPW;     // loads per lane per step (K and V, or Q)
+    constexpr int QS = 64 / BN;      // Q steps per query tile
+    constexpr int RQ = 32 / QS;      // query rows per wave and Q step
     static_assert(UPW >= 1 && TILE % (8 * 64 * 4) == 0, "tile must split into 1 KB wave loads");
+    static_assert(64 % BN == 0 && RQ * CPR == LPS * 64, "a Q step must load as much as a K/V step");
 
     __shared__ __attribute__((aligned(16))) __bf16 ring[NS][2][TILE];
 
@@ -100,7 +102,9 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     };
 
     // DMA geometry. K/V: wave-load j of this wave fills units [(wave * UPW + j) * 64, +64) of a
-    // tile; unit u holds key u / CPR, global 16-byte column (u % CPR) ^ swz(key).
+    // tile; unit u holds key u / CPR, global 16-byte column (u % CPR) ^ swz(key). Q step i: the
+    // wave's own RQ rows (rows 32 rb + RQ i + r of its head) fill its region of the stage,
+    // unit j * 64 + lane holding row r = unit / CPR, column (unit % CPR) ^ swz(r).
     int koff[UPW], voff[UPW];
 #pragma unroll
     for (int j = 0; j < UPW; ++j) {
@@ -110,7 +114,7 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
         voff[j] = key * v_row + ch * 16;
     }
     const uint32_t ring_base = uniform((int)lds_addr(&ring[0][0][0]));
-    constexpr uint32_t kStageBytes = 2 * TILE * 2, kTileBytes = TILE * 2;
+    constexpr uint32_t kStageBytes = 2 * TILE * 2, kTileBytes = TILE * 2, kQWaveBytes = RQ * D * 2;
     static_assert(LPS % 4 == 0 && UPW % 2 == 0, "loads go out four at a time");
     // LPS loads of one step (lds[i], voff[i]); the first UPW read through ra, the rest rb.
     auto dma_step = [&](const uint32_t (&lds)[LPS], const int (&off)[LPS], __amdgpu_buffer_rsrc_t ra,
@@ -136,8 +140,27 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
         }
         dma_step(lds, off, k_rs, v_rs);
     };
-    // Per-lane LDS read offsets (elements within a tile). K: key 32b + col, unit 2c + kg. V^T
-    // (tr16): in 16-lane group
+    // Q offsets are recomputed at each (rare) Q step rather than held in registers: the empty
+    // asm keeps the compiler from hoisting them out of the loop.
+    auto issue_q = [&](int stage, int qt, int i) {
+        const uint32_t qb = ring_base + stage * kStageBytes + wave * kQWaveBytes;
+        const int base = (qt * BM + rb * 32 + i * RQ) * q_row;
+        int ql = lane;
+        asm volatile("" : "+v"(ql));
+        uint32_t lds[LPS];
+        int off[LPS];
+#pragma unroll
+        for (int j = 0; j < LPS; ++j) {
+            const int u = j * 64 + ql;
+            const int r = u / CPR, ch = (u % CPR) ^ swz<CPR>(r);
+            lds[j] = qb + j * 1024;
+            off[j] = base + r * q_row + ch * 16;
+        }
+        dma_step(lds, off, q_rs, q_rs);
+    };
+
+    // Per-lane LDS read offsets (elements within a tile). K: key 32b + col, unit 2c + kg (the
+    // wave's Q rows use the same pattern: row col of its region). V^T (tr16): in 16-lane group
     // g = lane / 16, source lane i = lane % 16 points at key 16h + 4 * (g / 2) + i / 4 (+ 8 for
     // the second half of the operand) and dims 32 db + 16 (g % 2) + 4 (i % 4); the transpose
     // hands lane (m = dim, kg) four keys of its dim. Both swizzles depend only on bits of the
@@ -172,7 +195,7 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     };
     const float c2 = p.c;
 
-    // Current query tile.
+    // Current query tile; t < 0 marks its Q steps.
     int qt = qt_first, klo, ntiles;
     key_range(qt, klo, ntiles);
     int r0 = qt * BM + rb * 32;
@@ -180,16 +203,9 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     bool wave_active = r0 < L;
     int wr1 = min(L, r0 + 32);
     bf16x8 qf[DC];
+#pragma unroll
+    for (int c = 0; c < DC; ++c) qf[c] = bf16x8{};
     reset();
-    // The tile's query fragment (row col, dims 16 c + 8 kg .. + 7), straight into registers. The
-    // empty asm keeps the compiler's wait for it here, outside the step loop.
-    auto load_q = [&]() {
-        const int base = (r0 + col) * q_row + 16 * kg;
-#pragma unroll
-        for (int c = 0; c < DC; ++c) qf[c] = buf_ld16(q_rs, base + 32 * c, 0);
-#pragma unroll
-        for (int c = 0; c < DC; ++c) asm volatile("" : "+v"(qf[c]));
-    };
 
     // Step bookkeeping: `adv` moves a cursor one step ahead.
     struct Cursor {
@@ -198,29 +214,31 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     auto adv = [&](Cursor &c) {
         if (++c.t >= c.ntiles) {
             ++c.qt;
-            c.t = 0;
+            c.t = -QS;
             if (c.qt < qt_end) key_range(c.qt, c.klo, c.ntiles);
         }
     };
+    auto issue_step = [&](int stage, const Cursor &c) {
+        if (c.t < 0) issue_q(stage, c.qt, c.t + QS);
+        else issue_kv(stage, c.klo + c.t * BN);
+    };
 
-    // Prologue: every stage is free, so the first NS K/V tiles go out, then the query fragment,
-    // whose wait covers them too: one memory latency for the workgroup's start. (With the query
-    // rows as a step of the ring the first K/V tile went out only after they had landed: 5 %
-    // slower on 32 documents of median 700 tokens, 32:8 heads, 272 -> 258 us causal, 379 -> 365 us
-    // global; 1 % on 8 x 4,096.)
-    Cursor ld{qt, 0, klo, ntiles};  // next step to issue
+    // Prologue: issue the first NS - 1 steps. (Query rows straight into registers, behind the first NS
+    // K/V tiles and one wait, were measured and dropped: 1 to 2 % faster on most causal and global
+    // calls, 2 x 8,000 at 32:8 heads 1,303 -> 1,294 us, but slower where a tile has few key tiles:
+    // +-64 at 8 heads, 8 x 4,096, 69.2 -> 74.2 us; gated causal 16:2, 256 x U{65..200}, 120.8 -> 126.1.)
+    Cursor ld{qt, -QS, klo, ntiles};  // next step to issue
     int issued = 0;
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
+    for (int s = 0; s < NS - 1; ++s) {
         if (ld.qt < qt_end) {
-            issue_kv(issued % NS, ld.klo + ld.t * BN);
+            issue_step(issued % NS, ld);
             ++issued;
             adv(ld);
         }
     }
-    load_q();
 
-    int t = 0, step = 0;
+    int t = -QS, step = 0;
     while (true) {
         // This step's loads are complete once at most the later steps' loads are in flight
         // (loads complete in issue order; other outstanding accesses only make this stricter).
@@ -230,15 +248,28 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
         else wait_vmcnt<0>();
         __syncthreads();
         // Refill the stage freed by the previous step (all waves passed the barrier after it).
-        if (step > 0 && ld.qt < qt_end) {
-            issue_kv(issued % NS, ld.klo + ld.t * BN);
+        if (ld.qt < qt_end) {
+            issue_step(issued % NS, ld);
             ++issued;
             adv(ld);
         }
 
         const __bf16 *kt = &ring[step % NS][0][0];
+        if (t < 0) {
+            // Q step t + QS: lanes whose row is in this step's part read their fragments; the
+            // empty asm ends the reads' scope before the next barrier frees the stage.
+            const int i = t + QS;
+            if (QS == 1 || col / RQ == i) {
+                const __bf16 *qs = kt + wave * RQ * D - i * RQ * D;
+#pragma unroll
+                for (int c = 0; c < DC; ++c) qf[c] = ld_s16(qs + kbase_c[c]);
+#pragma unroll
+                for (int c = 0; c < DC; ++c) asm volatile("" : "+v"(qf[c]));
+            }
+        }
+
         const __bf16 *vt = &ring[step % NS][1][0];
-        if (wave_active) {
+        if (t >= 0 && wave_active) {
             const int kt0 = klo + t * BN;
             f32x16 s[NB];
             bool live[NB];
@@ -300,7 +331,7 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
             }
         }
 
-        if (t + 1 >= ntiles) {
+        if (t >= 0 && t + 1 >= ntiles) {
             // Last key tile of this query tile: normalise, apply the gate, store, reset.
             const float lsum = (ls[0] + ls[1]) + (ls[2] + ls[3]);
             const float lt = lsum + __shfl_xor(lsum, 32);
@@ -319,8 +350,7 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
             myrow = r0 + col;
             wave_active = r0 < L;
             wr1 = min(L, r0 + 32);
-            load_q();  // waits here (and for the ring's loads in flight): strips of several tiles only
-            t = 0;
+            t = -QS;
         } else {
             ++t;
         }
