@@ -456,4 +456,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_pe_torch", "Native launches of th
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__pe_torch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__pe_torch() {
+    if (pe_attn_abi_version() != PE_ATTN_ABI_VERSION) {
+        PyErr_Format(PyExc_ImportError, "_pe_torch was built for ABI %d of libpe_attn.so, which has %d", PE_ATTN_ABI_VERSION,
+                     pe_attn_abi_version());
+        return nullptr;
+    }
+    return PyModule_Create(&module);
+}

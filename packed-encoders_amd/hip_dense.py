@@ -3,7 +3,7 @@
 ``layer_norm``, ``add_layer_norm`` and ``geglu`` take the tensors of ``ops``' functions of the same
 names and return None for a call the kernels do not serve (``csrc/pe_torch.cpp`` says which), which
 ``ops`` then runs in torch; so does every call while torch compiles, or without a built library
-(the ``"sdpa"`` backend works without one).
+and extension (the ``"sdpa"`` backend works without either).
 """
 
 from __future__ import annotations

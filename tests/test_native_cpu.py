@@ -1,7 +1,12 @@
-"""What the layer's functions do where no native launch is possible: recorded calls (CPU only)."""
+"""What the layer's functions do where no native launch is possible: recorded calls, and a library
+without its extension (CPU only)."""
 
 from __future__ import annotations
 
+import sys
+import warnings
+
+import pytest
 import torch
 import torch.nn.functional as F
 
@@ -42,3 +47,21 @@ def test_layer_functions_compile_as_torchscript(pe):
     s, n = add(x, r, w, 1e-5)
     assert torch.equal(s, x + r) and torch.equal(n, want) and torch.equal(norm(x + r, w, 1e-5), want)
     assert torch.equal(gate(x), F.gelu(x[:, :16]) * x[:, 16:])
+
+
+def test_a_library_without_its_extension_warns_once(pe, monkeypatch):
+    """No ``_pe_torch.so`` beside a built library: no error, the general path, one warning."""
+    native = sys.modules[pe.__name__ + "._native"]
+    if not native.LIBRARY.exists():
+        pytest.skip("the library is not built")
+    monkeypatch.setitem(sys.modules, pe.__name__ + "._pe_torch", None)  # its import fails
+    monkeypatch.delattr(pe, "_pe_torch", raising=False)
+    native._module.cache_clear()
+    try:
+        with pytest.warns(RuntimeWarning, match="native launches are off"):
+            assert native._module() is None
+        with warnings.catch_warnings():
+            warnings.simplefilter("error")
+            assert native._module() is None
+    finally:
+        native._module.cache_clear()

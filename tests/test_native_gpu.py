@@ -175,3 +175,25 @@ def test_other_threads_run_during_a_launch(pe, name):
             thread.join()
         torch.cuda.synchronize()
     assert during > 0
+
+
+def test_calls_without_the_extension_take_the_general_path(pe, monkeypatch):
+    """A built library without ``_pe_torch.so``: the layer's norm and gate run in torch, attention
+    through the registered operators with the bits of the native launch."""
+    announce("calls without the extension")
+    native = sys.modules[pe.__name__ + "._native"]
+    x, w = torch.randn(40, 512, device="cuda").bfloat16(), torch.ones(512, device="cuda").bfloat16()
+    q, cu = torch.randn(40, 4, 64, device="cuda").bfloat16(), _cu([10, 30])
+    with torch.inference_mode():
+        want = pe.varlen_attention(q, q, q, cu, 30)
+        monkeypatch.setitem(sys.modules, pe.__name__ + "._pe_torch", None)
+        monkeypatch.delattr(pe, "_pe_torch", raising=False)
+        native._module.cache_clear()
+        try:
+            with pytest.warns(RuntimeWarning, match="native launches are off"):
+                got = pe.ops.layer_norm(x, w, 1e-5)
+            assert torch.equal(got, torch.nn.functional.layer_norm(x, (512,), w, None, 1e-5))
+            assert torch.equal(pe.ops.geglu(x), torch.nn.functional.gelu(x[:, :256]) * x[:, 256:])
+            assert torch.equal(pe.varlen_attention(q, q, q, cu, 30), want)
+        finally:
+            native._module.cache_clear()
