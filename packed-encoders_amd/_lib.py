@@ -118,8 +118,17 @@ def library(path: str | None = None) -> ctypes.CDLL:
         lib = ctypes.CDLL(str(lib_path))
     except OSError as exc:  # pragma: no cover - depends on the HIP runtime being present
         raise ImportError(f"cannot load {lib_path}: {exc}") from exc
-    lib.pe_attn_abi_version.restype = ctypes.c_int
-    lib.pe_attn_abi_version.argtypes = []
+    # The version first, then every symbol this package calls: a library built before one was added has
+    # the version but not the symbol, and is as stale as one of another version.
+    missing = [name for name in EXPORTED if not hasattr(lib, name)]
+    if EXPORTED[0] not in missing:
+        lib.pe_attn_abi_version.restype = ctypes.c_int
+        lib.pe_attn_abi_version.argtypes = []
+        version = lib.pe_attn_abi_version()
+        if version != ABI_VERSION:
+            raise ImportError(f"{lib_path} has ABI {version}, expected {ABI_VERSION}: rebuild it")
+    if missing:
+        raise ImportError(f"{lib_path} lacks {', '.join(missing)}: rebuild it")
     lib.pe_attn_strerror.restype = ctypes.c_char_p
     lib.pe_attn_strerror.argtypes = [ctypes.c_int]
     lib.pe_attn_workspace_size.restype = ctypes.c_int
@@ -152,9 +161,6 @@ def library(path: str | None = None) -> ctypes.CDLL:
                                       ctypes.c_void_p]
     lib.pe_geglu_fwd.restype = ctypes.c_int
     lib.pe_geglu_fwd.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_void_p]
-    version = lib.pe_attn_abi_version()
-    if version != ABI_VERSION:
-        raise ImportError(f"{lib_path} has ABI {version}, expected {ABI_VERSION}: rebuild it")
     return lib
 
 

@@ -1,8 +1,10 @@
-"""What the layer's functions do where no native launch is possible: recorded calls, and a library
-without its extension (CPU only)."""
+"""What the layer's functions do where no native launch is possible: recorded calls, a library
+without its extension, a stale library (CPU only)."""
 
 from __future__ import annotations
 
+import shutil
+import subprocess
 import sys
 import warnings
 
@@ -65,3 +67,18 @@ def test_a_library_without_its_extension_warns_once(pe, monkeypatch):
             assert native._module() is None
     finally:
         native._module.cache_clear()
+
+
+@pytest.mark.parametrize("version", [None, 8, 9])
+def test_a_stale_library_is_an_import_error(pe, tmp_path, version):
+    """A library of another ABI, or of this one but built before an entry point was added, is refused
+    as the loader promises, whatever it lacks."""
+    gcc = shutil.which("gcc")
+    if gcc is None:
+        pytest.skip("gcc is not available")
+    src, lib = tmp_path / "stale.c", tmp_path / "stale.so"
+    src.write_text("int pe_other(void) { return 0; }\n" if version is None
+                   else f"int pe_attn_abi_version(void) {{ return {version}; }}\n")
+    subprocess.run([gcc, "-shared", "-fPIC", str(src), "-o", str(lib)], check=True)
+    with pytest.raises(ImportError, match="rebuild it"):
+        pe._lib.library.__wrapped__(str(lib))
