@@ -46,14 +46,14 @@ bool plain_thread() {
 }
 
 // A dense tensor on the current HIP device that records nothing and is what it says (no subclass,
-// wrapper, lazy conjugation or forward derivative).
+// wrapper, batched stand-in without storage, lazy conjugation or forward derivative).
 bool plain_any(PyObject *obj, const Tensor *&out, at::ScalarType type) {
     if (!THPVariable_CheckExact(obj)) return false;
     const Tensor &t = THPVariable_Unpack(obj);
     static const c10::DispatchKeySet wrapped({DispatchKey::FuncTorchGradWrapper, DispatchKey::FuncTorchBatched,
                                               DispatchKey::Functionalize, DispatchKey::Python, DispatchKey::Conjugate,
                                               DispatchKey::Negative, DispatchKey::ZeroTensor});
-    if (!t.defined() || !t.is_cuda() || t.scalar_type() != type || t.layout() != at::kStrided ||
+    if (!t.defined() || !t.has_storage() || !t.is_cuda() || t.scalar_type() != type || t.layout() != at::kStrided ||
         t.key_set().has_any(wrapped) || t.get_device() != c10::hip::current_device())
         return false;
     if (t.requires_grad() && c10::GradMode::is_enabled()) return false;

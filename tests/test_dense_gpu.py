@@ -110,6 +110,26 @@ def test_other_calls_run_in_torch(pe):
     assert torch.equal(batched, each)
 
 
+def test_batched_derivatives_reach_the_torch_operations(pe):
+    """The batching that ``is_grads_batched`` and vectorised derivatives use hands backward functions
+    tensors without storage: they go to torch, as those of ``torch.func.vmap`` do."""
+    announce("batched derivatives")
+    w = _bf16(768)
+
+    class Gate(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x):
+            return x.clone()
+
+        @staticmethod
+        def backward(ctx, grad):
+            return pe.ops.layer_norm(grad, w, 1e-5)
+
+    x, grads = _bf16(4, 768).requires_grad_(), _bf16(3, 4, 768, seed=1)
+    got = torch.autograd.grad(Gate.apply(x), x, grads, is_grads_batched=True)[0]
+    assert torch.equal(got, F.layer_norm(grads, (768,), w, None, 1e-5))
+
+
 @pytest.mark.parametrize("d,theta", [(64, 160000.0), (64, 10000.0), (128, 10000.0), (256, 500.0)])
 def test_rope_rows_are_the_gathered_tables(pe, d, theta):
     announce(f"rope rows d={d} theta={theta}")
