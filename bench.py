@@ -135,7 +135,9 @@ def useful_flops_served(workload, short_max, kernel):
 
 def kernel_instance(lib, call, workload):
     """The name rocprofv3 lists (template arguments included) for the kernels of one layer's
-    call, as the library reports its choice (pe_attn_kernels): (short kernel, long kernel)."""
+    call, as the library reports its choice (pe_attn_kernels): (short kernel, long kernel). LayerCall
+    launches the stages over a shared plan, so its long kernel is the unsplit, planned instance (the
+    last two arguments false)."""
     from packed_encoders_amd import _lib
 
     out = (ctypes.c_int32 * 6)()

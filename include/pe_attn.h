@@ -201,11 +201,15 @@ int pe_packed_short_attn_fwd(const pe_attn_args *args, hipStream_t stream);
    (packed_encoders/_kernels/triton_packed_attention.py:29-42). */
 int pe_attn_short_config(int32_t max_seqlen, int32_t head_dim, int32_t out[4]);
 
-/* The kernels pe_varlen_attn_fwd runs for these arguments (host-only, like the workspace
-   size): out[0] the short kernel's key capacity (0: no short kernel), out[1] the long-segment
-   kernel (PE_ATTN_KERNEL_*), out[2] its query tiles per workgroup (strip), out[3] its query
+/* The kernels pe_varlen_attn_fwd runs for these arguments with a workspace of
+   pe_attn_workspace_size (host-only, like it): out[0] the short kernel's key capacity (0: no short
+   kernel, as in a split call with short_max -1), out[1] the long-segment kernel
+   (PE_ATTN_KERNEL_*), out[2] its query tiles per workgroup (strip), out[3] its query
    rows per tile, out[4] the short kernel's query heads per workgroup (fewer than
-   pe_attn_short_config's when the batch would leave CUs idle) and out[5] its workgroups.
+   pe_attn_short_config's when the batch would leave CUs idle, or with RoPE tables from 64 keys on)
+   and out[5] its workgroups. The long-segment kernel's instance is not told apart: key chunks
+   (pe_attn_key_chunks), or tiles it finds by itself where a plan costs more than it gives (narrow
+   windows and small split calls; the staged entry points always run it unsplit over their plan).
    No counterpart in the reference; for profiling and tests. */
 #define PE_ATTN_KERNEL_NONE 0
 #define PE_ATTN_KERNEL_TILED 1    /* tiled_attn_kernel: head_dim 64 windowed or causal */

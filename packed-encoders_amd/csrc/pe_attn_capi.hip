@@ -605,12 +605,15 @@ int launch_norm(const pe::NormParams &p, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? PE_ATTN_OK : PE_ATTN_ELAUNCH;
 }
 
-// A call split into key chunks. By default its short segments take the split kernel as well, which
-// serves any length: that spares the short pass, 4.7 us of a 92 us call that has none of them.
+// The boundary a split call routes by. By default its short segments take the split kernel as well,
+// which serves any length: that spares the short pass, 4.7 us of a 92 us call that has none of them.
+int split_short_max(const pe_attn_args *a) { return a->short_max < 0 ? 0 : a->short_max; }
+
+// A call split into key chunks.
 int launch_split(const pe_attn_args *call, const Split &split, void *workspace, size_t workspace_bytes,
                  hipStream_t stream) {
     pe_attn_args a = *call;
-    if (a.short_max < 0) a.short_max = 0;
+    a.short_max = split_short_max(&a);
     a.max_seqlen_k = longest_keys(&a);  // what the partial rows are sized for: a longer segment is skipped
     Plan plan;
     int rc = prepare(&a, &plan);
@@ -759,7 +762,9 @@ int pe_attn_kernels(const pe_attn_args *a, int32_t out[6]) {
     int rc = check_args(a, false);
     if (rc) return rc;
     if (!out) return PE_ATTN_EINVAL;
-    const int sm = effective_short_max(a);
+    pe_attn_args routed = *a;
+    if (pe_attn_key_chunks(a) > 1) routed.short_max = split_short_max(a);
+    const int sm = effective_short_max(&routed);
     int sk = 0, heads = 0;
     if (sm > 0) short_launch_shape(sm, a->head_dim, a->rope_cos != nullptr, a->n_seq, a->n_heads_q, &sk, &heads);
     const int g = heads_per_tile(a);

@@ -409,3 +409,21 @@ def test_min_seqlen_above_the_boundary_skips_the_short_pass(lib):
     assert _kernels(lib, max_seqlen=64, min_seqlen=64) == (64, _lib.KERNEL_NONE, 0, 0)
     rc, size = _ws(lib, _args(min_seqlen=98))
     assert rc == 0 and size == 256 + 16 * min(64 * 8, (32438 + 64 * 255) // 256)
+
+
+def test_kernel_choice_of_a_split_call(lib):
+    """A split call routes nothing to the short kernel unless it was asked to, and pe_attn_kernels says
+    so; the same call with its keys unsplit (a key bound too short to split) still has its short pass."""
+    kw = dict(n_seq=8, total_tokens=128, max_seqlen=16, n_heads_q=32, n_heads_kv=8, head_dim=128, causal=1)
+
+    def kernels(short_max, keys):
+        out = (ctypes.c_int32 * 6)()
+        a = _args(short_max=short_max, **kw)
+        a.cu_seqlens_k, a.total_tokens_k, a.max_seqlen_k = 8, 8 * keys, keys  # sizes only
+        assert lib.pe_attn_kernels(ctypes.byref(a), out) == 0
+        return lib.pe_attn_key_chunks(ctypes.byref(a)) > 1, out[0], out[4], out[5]
+
+    assert kernels(-1, 4096) == (True, 0, 0, 0)
+    assert kernels(0, 4096) == (True, 0, 0, 0)
+    assert kernels(32, 4096) == (True, 32, 1, 8 * 32)
+    assert kernels(-1, 1000) == (False, 32, 1, 8 * 32)
