@@ -134,9 +134,15 @@ int pe_attn_abi_version(void);
 const char *pe_attn_strerror(int status);
 
 /* Bytes of device workspace pe_varlen_attn_fwd needs for these arguments (host-only, from
-   n_seq, total_tokens, max_seqlen, min_seqlen, head geometry and short_max; never reads
-   device memory). */
+   n_seq, total_tokens, max_seqlen, min_seqlen, head geometry, window, causal, short_max, strip,
+   band_kernel and the key segments' total_tokens_k and max_seqlen_k; never reads device memory): the
+   list of pe_attn_plan and, for a call whose keys are split (pe_attn_key_chunks), its partial rows, up
+   to 256 MiB. */
 int pe_attn_workspace_size(const pe_attn_args *args, size_t *bytes);
+
+/* The part of pe_attn_workspace_size that the staged entry points use, the list alone: pe_attn_plan
+   and pe_attn_tiled_fwd need no more, and pe_varlen_attn_fwd runs unsplit with it. Host-only. */
+int pe_attn_plan_size(const pe_attn_args *args, size_t *bytes);
 
 /* The chunks pe_varlen_attn_fwd cuts the longest key segment into when it spreads a call's key
    segments over workgroups of their own (few query rows against long cu_seqlens_k segments), 1 when

@@ -24,6 +24,7 @@ EXPORTED = (
     "pe_attn_abi_version",
     "pe_attn_strerror",
     "pe_attn_workspace_size",
+    "pe_attn_plan_size",
     "pe_attn_key_chunks",
     "pe_varlen_attn_fwd",
     "pe_varlen_attn_fwd_noalloc",
@@ -133,6 +134,8 @@ def library(path: str | None = None) -> ctypes.CDLL:
     lib.pe_attn_strerror.argtypes = [ctypes.c_int]
     lib.pe_attn_workspace_size.restype = ctypes.c_int
     lib.pe_attn_workspace_size.argtypes = [ctypes.POINTER(AttnArgs), ctypes.POINTER(ctypes.c_size_t)]
+    lib.pe_attn_plan_size.restype = ctypes.c_int
+    lib.pe_attn_plan_size.argtypes = [ctypes.POINTER(AttnArgs), ctypes.POINTER(ctypes.c_size_t)]
     lib.pe_attn_key_chunks.restype = ctypes.c_int
     lib.pe_attn_key_chunks.argtypes = [ctypes.POINTER(AttnArgs)]
     lib.pe_varlen_attn_fwd.restype = ctypes.c_int

@@ -659,6 +659,14 @@ int pe_attn_workspace_size(const pe_attn_args *a, size_t *bytes) {
     return PE_ATTN_OK;
 }
 
+int pe_attn_plan_size(const pe_attn_args *a, size_t *bytes) {
+    if (!bytes) return PE_ATTN_EINVAL;
+    const int rc = check_args(a, false);
+    if (rc) return rc;
+    *bytes = list_bytes(capacity_of(a));
+    return PE_ATTN_OK;
+}
+
 int pe_attn_key_chunks(const pe_attn_args *a) {
     const int rc = check_args(a, false);
     if (rc) return rc;
@@ -725,7 +733,7 @@ int pe_varlen_attn_fwd_noalloc(const pe_attn_args *a, hipStream_t stream) {
     int rc = pe_attn_workspace_size(a, &need);
     if (rc) return rc;
     // Where the partial rows of a split do not fit, the list alone: the call then runs unsplit.
-    if (need > PE_ATTN_STATIC_SCRATCH_BYTES) need = list_bytes(capacity_of(a));
+    if (need > PE_ATTN_STATIC_SCRATCH_BYTES && (rc = pe_attn_plan_size(a, &need))) return rc;
     if (need > PE_ATTN_STATIC_SCRATCH_BYTES) return PE_ATTN_ESCRATCH;
     void *ws = nullptr;
     if (need > 0 && (rc = static_scratch(&ws))) return rc;

@@ -146,7 +146,7 @@ def _run_planned(lib, plans: dict, args: _lib.AttnArgs, cu: Tensor, cu_k: Tensor
     ref = ctypes.byref(args)
     if entry is None:
         size = ctypes.c_size_t(0)
-        _lib.check(lib.pe_attn_workspace_size(ref, ctypes.byref(size)), "pe_attn_workspace_size")
+        _lib.check(lib.pe_attn_plan_size(ref, ctypes.byref(size)), "pe_attn_plan_size")
         workspace = torch.empty(size.value, dtype=torch.uint8, device=cu.device) if size.value else None
         ptr = workspace.data_ptr() if workspace is not None else None
         _lib.check(lib.pe_attn_plan(ref, ptr, size.value, stream), "pe_attn_plan")

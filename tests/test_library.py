@@ -427,3 +427,18 @@ def test_kernel_choice_of_a_split_call(lib):
     assert kernels(0, 4096) == (True, 0, 0, 0)
     assert kernels(32, 4096) == (True, 32, 1, 8 * 32)
     assert kernels(-1, 1000) == (False, 32, 1, 8 * 32)
+
+
+def test_plan_size_is_the_list_alone(lib):
+    """The staged entry points never read a split call's partial rows, and are not asked for them."""
+    def plan(a):
+        size = ctypes.c_size_t()
+        assert lib.pe_attn_plan_size(ctypes.byref(a), ctypes.byref(size)) == 0
+        return size.value
+
+    assert plan(_args()) == _ws(lib, _args())[1] > 0 and plan(_args(max_seqlen=64)) == 0
+    a = _args(n_seq=8, total_tokens=128, max_seqlen=16, n_heads_q=32, n_heads_kv=8, head_dim=128, causal=1)
+    a.cu_seqlens_k, a.total_tokens_k, a.max_seqlen_k = 8, 8 * 4096, 4096  # sizes only
+    assert lib.pe_attn_key_chunks(ctypes.byref(a)) > 1
+    assert plan(a) == 256 + 16 * 8 < _ws(lib, a)[1]
+    assert lib.pe_attn_plan_size(ctypes.byref(a), None) == lib.pe_attn_plan_size(None, ctypes.c_size_t()) == -1

@@ -213,3 +213,27 @@ def test_split_call_under_a_loose_bound(pe, d):
                                   max_seqlen_k=1 << 20)
     want = pe.runtime_attention.oracle_attention(q, k, v, TAILS, KEYS, True)
     assert (got.double() - want).abs().max() <= 2e-2
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[3], CASES[6]], ids=str)
+def test_staged_call_needs_the_plan_alone(pe, case):
+    """The staged entry points over a workspace of pe_attn_plan_size, and the whole call with it: unsplit,
+    bit for bit alike."""
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    announce(f"staged call over the plan alone {case}")
+    d, hq, hkv, window, causal, gated = case
+    q, k, v, gate = _inputs(d, hq, hkv, gated, seed=d)
+    lib, cu, cuk, out = _lib.library(), _cu(TAILS), _cu(KEYS), torch.full_like(q, 7.0)
+    a = _args(q, k, v, out, cu, max(TAILS), d ** -0.5, *window, causal, gate, 0, cu_k=cuk, max_seqlen_k=max(KEYS))
+    size, ref, stream = ctypes.c_size_t(), ctypes.byref(a), torch.cuda.current_stream().cuda_stream
+    assert lib.pe_attn_plan_size(ref, ctypes.byref(size)) == 0 and lib.pe_attn_key_chunks(ref) > 1
+    guard = torch.full((size.value + 4096,), 0xAA, dtype=torch.uint8, device="cuda")
+    assert lib.pe_attn_plan(ref, guard.data_ptr(), size.value, stream) == 0
+    assert lib.pe_attn_short_fwd(ref, stream) == 0
+    assert lib.pe_attn_tiled_fwd(ref, guard.data_ptr(), size.value, stream) == 0
+    torch.cuda.synchronize()
+    assert (guard[size.value:] == 0xAA).all()
+    whole = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda chunks, n: size.value, 0)
+    assert torch.equal(out, whole)
