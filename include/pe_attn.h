@@ -169,8 +169,11 @@ int pe_varlen_attn_fwd(const pe_attn_args *args, void *workspace, size_t workspa
    that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that
    forbid hipMalloc). No counterpart in the reference. It calls no allocating routine; its first
    call on a device looks the array's device address up once (hipGetSymbolAddress).
-   Returns PE_ATTN_ESCRATCH, launching nothing, when pe_attn_workspace_size exceeds the array
-   (at 1 MiB: about 65,000 (segment, query tile) entries). Every call on one GPU shares that
+   Returns PE_ATTN_ESCRATCH, launching nothing, when pe_attn_plan_size exceeds the array
+   (at 1 MiB: about 65,000 (segment, query tile) entries). The result is pe_varlen_attn_fwd's bit for
+   bit where pe_attn_workspace_size fits the array; a call whose keys would be split into partial
+   rows that do not fit runs unsplit, in the unsplit call's time and with its bits, which agree with
+   the split call's within rounding. Every call on one GPU shares that
    GPU's array: calls that overlap on one GPU (other streams, other threads) race and must be
    serialised by the caller. */
 #define PE_ATTN_STATIC_SCRATCH_BYTES (1u << 20)

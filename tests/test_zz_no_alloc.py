@@ -5,7 +5,8 @@ The variant keeps the tiled kernels' plan list in the library's static device ar
 of a caller workspace. Two calls in a row, the second with a smaller input, must each give
 bit-identical outputs to the workspace entry point (the second call reuses the array the
 first one filled, so stale entries must not leak into it); the short kernel's segments and
-all three head dims are covered.
+all three head dims are covered. A call whose keys the workspace entry point splits, with partial rows
+that do not fit the array, gives the unsplit call's bits instead.
 """
 
 from __future__ import annotations
@@ -196,6 +197,38 @@ def test_noalloc_captured_replays_follow_rewritten_lengths(pe):
         n = int(cus[i][-1])
         assert torch.equal(out[:n], want[:n]), f"replay with lengths {batches[i]} differs"
     del graph
+
+
+@pytest.mark.parametrize("d,n,fits", [(64, 1, True), (128, 1, True), (256, 1, True), (64, 8, False), (128, 8, False),
+                                      (256, 8, False)])
+def test_noalloc_of_split_calls(pe, d, n, fits):
+    """A few rows against long key segments: split as the workspace entry point splits them where the
+    partial rows fit the array, else unsplit (the workspace entry point over the plan's bytes alone)."""
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    announce(f"noalloc split d={d} n={n}")
+    lib, (hq, hkv), tail = _lib.library(), (4, 2), 1 if fits else 64
+    keys = [3000 - 37 * i for i in range(n)]
+    g = torch.Generator().manual_seed(d + n)
+    q, k, v = (torch.randn(t, h, d, generator=g).bfloat16().cuda()
+               for t, h in ((n * tail, hq), (sum(keys), hkv), (sum(keys), hkv)))
+    cu, cuk = (torch.tensor([0, *np.cumsum(x).tolist()], dtype=torch.int32, device="cuda") for x in ([tail] * n, keys))
+    outs = [torch.full_like(q, 5.0) for _ in range(2)]
+    calls = [_args(q, k, v, o, cu, tail, d ** -0.5, -1, -1, True, None, 0, cu_k=cuk, max_seqlen_k=max(keys)) for o in outs]
+    size, stream = ctypes.c_size_t(), torch.cuda.current_stream().cuda_stream
+    assert lib.pe_attn_key_chunks(ctypes.byref(calls[0])) > 1
+    assert lib.pe_attn_workspace_size(ctypes.byref(calls[0]), ctypes.byref(size)) == 0
+    assert (size.value <= _lib.STATIC_SCRATCH_BYTES) == fits, size.value
+    if not fits:
+        assert lib.pe_attn_plan_size(ctypes.byref(calls[0]), ctypes.byref(size)) == 0
+    ws = torch.full((size.value,), 0xFF, dtype=torch.uint8, device="cuda")
+    assert lib.pe_varlen_attn_fwd(ctypes.byref(calls[0]), ws.data_ptr(), size.value, stream) == 0
+    assert lib.pe_varlen_attn_fwd_noalloc(ctypes.byref(calls[1]), stream) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(outs[1], outs[0])
+    want = pe.runtime_attention.oracle_attention(q, k, v, [tail] * n, keys, True)
+    assert (outs[1].double() - want).abs().max() <= 2e-2
 
 
 _CHILD = r"""
