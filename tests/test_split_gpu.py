@@ -131,6 +131,79 @@ def test_split_call_of_many_segments_is_planned(pe):
         got = pe.varlen_attention(q, k, v, _cu(tails), 2, causal=True, cu_seqlens_k=_cu(keys), max_seqlen_k=2100)
     want = pe.runtime_attention.oracle_attention(q, k, v, tails, keys, True)
     assert (got.double() - want).abs().max() <= 2e-2
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    a = _args(q, k, v, got, _cu(tails), 2, 128 ** -0.5, -1, -1, True, None, -1, cu_k=_cu(keys), max_seqlen_k=2100)
+    assert _lib.library().pe_attn_key_chunks(ctypes.byref(a)) > 1  # it did split
+
+
+def _edge_batch(d, hq, hkv, n, chunk):
+    """Tails and key lengths of n segments whose call is cut into chunks of `chunk` keys: segments at the
+    chunk's edges, none, few and many keys, and the others sized so that the rule gives that chunk."""
+    g = np.gcd(hq // hkv, 4)
+    bm = (64 if d == 256 else 128) // g
+    groups, slots = n * hq // g, (3 if d == 64 else 2) * 256
+    mean = (chunk - 32) * (slots * 7 // 4 - groups) // (2 * groups)
+    edges = [chunk - 1, chunk, chunk + 1, 2 * chunk - 1, 2 * chunk, 2 * chunk + 1, 0, 1, 63, 65, max(1700, 3 * chunk)]
+    rng = np.random.default_rng(d + n + chunk)
+    rest = (mean - 1) * n - sum(edges)
+    assert rest > 0
+    others = rng.multinomial(rest, rng.dirichlet(np.full(n - len(edges), 8.0)))
+    order = rng.permutation(n)
+    keys = np.array(edges + others.tolist())[order]
+    tails = np.array([(bm, 1, bm - 1, 2, 5)[i % 5] for i in range(n - 1)] + [0])[order]
+    return keys.tolist(), tails.tolist()
+
+
+# head_dim, query heads, kv heads, segments (480 workgroups of the unsplit call), window, causal, gate
+EDGE_CASES = [
+    (64, 8, 8, 60, (-1, -1), True, True), (64, 8, 4, 120, (900, 900), False, False), (64, 8, 2, 240, (1700, -1), True, True),
+    (128, 8, 8, 60, (-1, -1), False, False), (128, 8, 4, 120, (-1, -1), True, True), (128, 8, 2, 240, (900, 900), False, True),
+    (256, 8, 8, 60, (1700, -1), True, False), (256, 8, 4, 120, (-1, -1), False, True), (256, 8, 2, 240, (-1, -1), True, False),
+]
+
+
+@pytest.mark.parametrize("chunk", [320, 640, 1152])
+@pytest.mark.parametrize("case", EDGE_CASES, ids=str)
+def test_split_instances_at_their_chunk_edges(pe, case, chunk):
+    """Every head_dim and heads per workgroup, gated and not, with chunks under 1,024 keys (the kernels
+    find their tiles) and past it (they read the plan, which the workspace's header tells)."""
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    d, hq, hkv, n, window, causal, gated = case
+    announce(f"split chunk {chunk} {case}")
+    keys, tails = _edge_batch(d, hq, hkv, n, chunk)
+    g = torch.Generator(device="cuda").manual_seed(d + chunk)
+    q, k, v, gt = (torch.randn(t, h, d, generator=g, device="cuda").bfloat16()
+                   for t, h in ((sum(tails), hq), (sum(keys), hkv), (sum(keys), hkv), (sum(tails), hq)))
+    lib, cu, cuk, stream = _lib.library(), _cu(tails), _cu(keys), torch.cuda.current_stream().cuda_stream
+    outs, header = [], None
+    for size_of in (lib.pe_attn_workspace_size, lib.pe_attn_plan_size):  # split, unsplit
+        out = torch.full_like(q, 7.0)
+        a = _args(q, k, v, out, cu, max(tails), d ** -0.5, *window, causal, gt if gated else None, 0, cu_k=cuk,
+                  max_seqlen_k=max(keys))
+        assert lib.pe_attn_key_chunks(ctypes.byref(a)) == -(-max(keys) // chunk) > 1
+        size = ctypes.c_size_t()
+        assert size_of(ctypes.byref(a), ctypes.byref(size)) == 0
+        ws = torch.full((size.value,), 0xFF, dtype=torch.uint8, device="cuda")  # unwritten partial rows are NaN
+        assert lib.pe_varlen_attn_fwd(ctypes.byref(a), ws.data_ptr(), size.value, stream) == 0
+        torch.cuda.synchronize()
+        outs.append(out)
+        header = ws[:8].view(torch.int32).tolist() if header is None else header
+    assert header == [-1, -1] if chunk < 1024 else header[0] == header[1] == sum(t > 0 for t in tails)
+    want = pe.runtime_attention.oracle_attention(q, k, v, tails, keys, causal, window)
+    if gated:
+        want = want * torch.sigmoid(gt.double())
+    at = 0
+    for tail, length in zip(tails, keys):
+        part = slice(at, at + tail)
+        if length <= chunk:
+            assert torch.equal(outs[0][part], outs[1][part]), (tail, length)
+        at += tail
+    for got in outs:
+        assert (got.double() - want).abs().max() <= 2e-2
 
 
 @pytest.mark.parametrize("d", [64, 128, 256])
