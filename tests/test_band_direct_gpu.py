@@ -1,8 +1,10 @@
 """Narrow-window calls that run without a plan, every workgroup finding its tile from cu_seqlens: the
 bits of the planned (staged) call over segment counts at the edges of the lanes' share, short, empty
-and over-long segments, heads and gates."""
+and over-long segments, heads and gates; and which calls run so."""
 
 from __future__ import annotations
+
+import ctypes
 
 import numpy as np
 import pytest
@@ -48,12 +50,9 @@ def test_direct_call_equals_the_planned_call(pe, n, hq, hkv, window, causal, gat
 
 def test_over_long_segments_stay_unwritten(pe):
     announce("direct band: a segment past max_seqlen")
-    lengths = [300, 900, 200]
     cu = torch.tensor([0, 300, 1200, 1400], dtype=torch.int32, device="cuda")
     q = torch.randn(1400, 4, 64, device="cuda").bfloat16()
     out = torch.full_like(q, 7.0)
-    import ctypes
-
     from packed_encoders_amd import _lib
     from packed_encoders_amd.hip_attention import _args
 
@@ -66,4 +65,41 @@ def test_over_long_segments_stay_unwritten(pe):
     assert lib.pe_varlen_attn_fwd(ctypes.byref(a), ws.data_ptr(), size.value, stream) == 0
     torch.cuda.synchronize()
     assert (out[300:1200] == 7.0).all() and not (out[:300] == 7.0).all() and not (out[1200:] == 7.0).all()
-    assert sum(lengths) == 1400
+
+
+# segments, tokens each, query heads, kv heads, head_dim, window, causal, strip, band_kernel: planless or planned
+FORMS = {
+    "one segment": ((1, 300, 4, 4, 64, (64, 64), False, 0, 0), True),
+    "256 segments": ((256, 130, 4, 4, 64, (64, 64), False, 0, 0), True),
+    "257 segments": ((257, 130, 4, 4, 64, (64, 64), False, 0, 0), False),
+    "window of 256 in all": ((4, 300, 4, 4, 64, (200, 56), False, 0, 0), True),
+    "window of 257 in all": ((4, 300, 4, 4, 64, (200, 57), False, 0, 0), False),
+    "causal, 256 to the left": ((4, 300, 4, 4, 64, (256, -1), True, 0, 0), True),
+    "one side unbounded": ((4, 300, 4, 4, 64, (64, -1), False, 0, 0), False),
+    "12,288 query tiles": ((1, 128 * 96, 128, 64, 64, (8, 8), False, 0, 0), True),
+    "12,416 query tiles": ((1, 128 * 97, 128, 64, 64, (8, 8), False, 0, 0), False),
+    "a strip of two": ((4, 300, 4, 4, 64, (64, 64), False, 2, 0), False),
+    "the band kernel": ((4, 300, 4, 4, 64, (64, 64), False, 0, 1), False),
+    "head_dim 128": ((4, 300, 4, 4, 128, (64, 64), False, 0, 0), False),
+}
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_which_calls_run_without_a_plan(pe, form):
+    """A plan writes the workspace's header, a planless call leaves it alone."""
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    announce(f"direct band: {form}")
+    (n, tokens, hq, hkv, d, window, causal, strip, band), direct = FORMS[form]
+    cu = torch.arange(0, (n + 1) * tokens, tokens, dtype=torch.int32, device="cuda")
+    q, k = (torch.randn(n * tokens, h, d, device="cuda").bfloat16() for h in (hq, hkv))
+    out = torch.empty_like(q)
+    a = _args(q, k, k, out, cu, tokens, 0.125, *window, causal, None, -1, strip, band_kernel=band)
+    lib, size = _lib.library(), ctypes.c_size_t()
+    assert lib.pe_attn_workspace_size(ctypes.byref(a), ctypes.byref(size)) == 0
+    ws = torch.full((size.value,), 0xFF, dtype=torch.uint8, device="cuda")
+    assert lib.pe_varlen_attn_fwd(ctypes.byref(a), ws.data_ptr(), size.value, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    written, needed = ws[:8].view(torch.int32).tolist()
+    assert (written, needed) == (-1, -1) if direct else written == needed > 0
