@@ -377,6 +377,23 @@ int launch_tiled_d(const AttnParams &p, int g, bool gate, int64_t cap, hipStream
     return win ? launch_tiled_g<D, false, true>(p, g, cap, stream) : launch_tiled_g<D, false, false>(p, g, cap, stream);
 }
 
+// How a split launch deals its workgroups to the XCDs (split_item): sets p.share and p.tiles, returns
+// the workgroups per chunk. Fewer than eight sets of keys are dealt one by one: each chunk then has its
+// XCDs to itself. Unsplit / dealt one by one / so, us, causal: 32 x U{1400..2500} keys, one row, 12:4 x 256
+// (three head groups a kv head) 90 / 121 / 63; 64 x the same, 12:2 x 128 (three) 68 / 75 / 59; 62 x
+// U{500..8000}, 64-row tails (four tiles), 8:2 x 256, 330 / 385 / 281.
+int64_t split_deal(AttnParams &p, int g, int64_t cap) {
+    p.share = p.group / g;
+    p.tiles = (int)((2 * cap + p.n_seq) / (2 * (int64_t)p.n_seq));
+    if (p.tiles < 1) p.tiles = 1;
+    const int64_t units = (cap + p.tiles - 1) / p.tiles * (p.hgroups / p.share), members = (int64_t)p.share * p.tiles;
+    if (members == 1 || units < 8) {
+        p.share = p.tiles = 1;
+        return cap * p.hgroups;
+    }
+    return (units + 7) / 8 * 8 * members;
+}
+
 // Split launches (pe_attn_split.h): one workgroup per work entry, head group and key chunk, then the
 // merge of every entry's rows.
 template <int D, int G, bool DIRECT>
@@ -385,7 +402,7 @@ int launch_split_t(AttnParams p, int bm, int64_t cap, int chunks, hipStream_t st
     p.hgroups = p.hq / G;
     // Workgroup i runs on XCD i % 8: one workgroup past a multiple of 8 per chunk spreads a segment's
     // chunks over the XCDs, which hold unequal shares of the keys otherwise.
-    const int64_t items = cap * p.hgroups;
+    const int64_t items = split_deal(p, G, cap);
     const dim3 grid((unsigned)(items + (9 - items % 8) % 8), chunks);
     if constexpr (D == 64)
         hipLaunchKernelGGL((pe::tiled_attn_kernel<D, G, BN, NS, false, true, true, DIRECT>), grid, dim3(256), 0, stream, p);

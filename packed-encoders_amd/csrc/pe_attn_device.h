@@ -62,6 +62,7 @@ struct AttnParams {
         struct {
             float *part_o, *part_ml;
             int32_t chunk, total_q;
+            int32_t share, tiles;  // head groups and work entries dealt to one XCD together (split_item)
         };
     };
 };
@@ -112,7 +113,8 @@ __device__ __forceinline__ int wave_scan(int x) {
 // last tiles (the cheaper ones, so that the launch ends on them). Lane l takes segments 4 l .. 4 l + 3
 // (at most kDirectSegments), a scan over the lanes numbers their tiles. For calls whose full tiles
 // all cost about the same; the same segments take tiles as in the plan (longer than short_max,
-// within the caller's bounds). KEYS: the key segments are the call's own (cuk).
+// within the caller's bounds). KEYS: the key segments are the call's own (cuk), and a segment's tiles,
+// which cost alike however few rows the last one has, stay together.
 constexpr int kDirectSegments = 256;
 
 template <bool KEYS = false>
@@ -134,7 +136,7 @@ __device__ __forceinline__ WorkItem find_work(const AttnParams &p, int entry, in
         } else {
             mine = mine && L > p.short_max;
         }
-        full[i] = mine ? L / bm : 0;
+        full[i] = mine ? (KEYS ? (L + bm - 1) / bm : L / bm) : 0;
         part[i] = mine && full[i] * bm < L ? 1 : 0;
         n_full += full[i];
         n_part += part[i];

@@ -15,6 +15,24 @@
 
 namespace pe {
 
+// The work entry and head group of a split call's workgroup. Those that read the same keys (the head
+// groups of one kv head, over the `tiles` consecutive entries that a segment has on average) go to one
+// XCD, eight workgroups apart, so that all but the first of them find the keys in that XCD's L2;
+// dealt one by one to the XCDs, each fetched them again (split_deal, pe_attn_capi.hip).
+__device__ __forceinline__ void split_item(const AttnParams &p, int &entry, int &hg) {
+    const int x = blockIdx.x, members = p.share * p.tiles;
+    if (members <= 1) {
+        entry = x / p.hgroups;
+        hg = x - entry * p.hgroups;
+        return;
+    }
+    const int round = x / (8 * members), r = x - round * 8 * members;
+    const int unit = round * 8 + (r & 7), member = r >> 3, kv_heads = p.hgroups / p.share;
+    const int block = unit / kv_heads, tile = member / p.share;
+    entry = block * p.tiles + tile;
+    hg = (unit - block * kv_heads) * p.share + member - tile * p.share;
+}
+
 // Place of a row's partials: (chunk, query row, head).
 __device__ __forceinline__ int64_t part_slot(const AttnParams &p, int chunk, int row, int qh) {
     return ((int64_t)chunk * p.total_q + row) * p.hq + qh;

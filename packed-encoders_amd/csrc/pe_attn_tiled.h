@@ -100,8 +100,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
         const int j = (int)(blockIdx.x >> 3);
         item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
     }
-    const int entry = item / p.hgroups;
-    const int hg = item - entry * p.hgroups;
+    int entry = item / p.hgroups;
+    int hg = item - entry * p.hgroups;
+    if constexpr (SPLIT) split_item(p, entry, hg);
     const WorkItem wi = DIRECT ? find_work<SPLIT>(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;

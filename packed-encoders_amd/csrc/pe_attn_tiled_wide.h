@@ -52,9 +52,10 @@ __global__ __launch_bounds__(256) void wide_attn_kernel(AttnParams p) {
     // XCD's L2 (dealt one item per XCD, every tile fetched them again from memory).
     const int rh = wide_run(p.hgroups);
     const int j = (int)(blockIdx.x >> 3);
-    const int item = SPLIT ? (int)blockIdx.x : ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
-    const int entry = item / p.hgroups;
-    const int hg = item - entry * p.hgroups;
+    const int item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
+    int entry = item / p.hgroups;
+    int hg = item - entry * p.hgroups;
+    if constexpr (SPLIT) split_item(p, entry, hg);
     const WorkItem wi = DIRECT ? find_work<SPLIT>(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;

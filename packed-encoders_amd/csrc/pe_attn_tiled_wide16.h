@@ -91,9 +91,10 @@ __global__ __launch_bounds__(64 * NW) void wide16_attn_kernel(AttnParams p) {
     // wide16_run() items dealt to the XCDs in turn).
     const int rh = wide16_run<NW, NS>(p.hgroups);
     const int j = (int)(blockIdx.x >> 3);
-    const int item = SPLIT ? (int)blockIdx.x : ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
-    const int entry = item / p.hgroups;
-    const int hg = item - entry * p.hgroups;
+    const int item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
+    int entry = item / p.hgroups;
+    int hg = item - entry * p.hgroups;
+    if constexpr (SPLIT) split_item(p, entry, hg);
     const WorkItem wi = DIRECT ? find_work<SPLIT>(p, entry, BM) : load_work(p, entry);
     if (!wi.valid) return;
     const int qt_first = wi.qt_first;

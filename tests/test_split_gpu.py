@@ -310,3 +310,29 @@ def test_staged_call_needs_the_plan_alone(pe, case):
     assert (guard[size.value:] == 0xAA).all()
     whole = _call(pe, case, q, k, v, gate, torch.full_like(q, 7.0), lambda chunks, n: size.value, 0)
     assert torch.equal(out, whole)
+
+@pytest.mark.parametrize("hq,hkv", [(8, 1), (12, 4), (12, 2), (5, 1), (8, 2)])
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_split_calls_whose_workgroups_share_keys(pe, d, hq, hkv):
+    """Head groups of one kv head (two, three, three, five, one) and tails of up to three query tiles, ragged and
+    empty ones among them: workgroups that share keys are dealt to one XCD, every row is written once."""
+    from packed_encoders_amd import _lib
+    from packed_encoders_amd.hip_attention import _args
+
+    bm = (64 if d == 256 else 128) // int(np.gcd(hq // hkv, 4))
+    lib, stream = _lib.library(), torch.cuda.current_stream().cuda_stream
+    for tails in ([1] * 11, [3 * bm, 2 * bm + 1, bm, 0, 3 * bm - 1, 1, 2 * bm, 2 * bm - 1, 3 * bm], [2 * bm] * 8):
+        announce(f"split, shared keys, head_dim {d}, heads {hq}:{hkv}, tails {tails}")
+        keys = [3000 - 211 * i for i in range(len(tails))]
+        g = torch.Generator(device="cuda").manual_seed(d + hq)
+        q, k, v = (torch.randn(t, h, d, generator=g, device="cuda").bfloat16()
+                   for t, h in ((sum(tails), hq), (sum(keys), hkv), (sum(keys), hkv)))
+        cu, cuk, out, size = _cu(tails), _cu(keys), torch.full_like(q, 7.0), ctypes.c_size_t()
+        a = _args(q, k, v, out, cu, max(tails), d ** -0.5, -1, -1, True, None, 0, cu_k=cuk, max_seqlen_k=max(keys))
+        assert lib.pe_attn_workspace_size(ctypes.byref(a), ctypes.byref(size)) == 0
+        assert lib.pe_attn_key_chunks(ctypes.byref(a)) > 1
+        ws = torch.full((size.value,), 0xFF, dtype=torch.uint8, device="cuda")  # unwritten partial rows are NaN
+        assert lib.pe_varlen_attn_fwd(ctypes.byref(a), ws.data_ptr(), size.value, stream) == 0
+        torch.cuda.synchronize()
+        want = pe.runtime_attention.oracle_attention(q, k, v, tails, keys, True)
+        assert (out.double() - want).abs().max() <= 2e-2
