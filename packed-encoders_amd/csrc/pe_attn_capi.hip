@@ -526,15 +526,15 @@ struct Split {
 // walks, from host-known sizes. The chunk is the smallest (256 to 1,536 keys, in whole key tiles)
 // at which the call's workgroups still fit the chip at once: smaller chunks add partial rows and
 // rounds of short-lived workgroups, larger ones leave it idle. A call of more than two unsplit
-// workgroups per CU stays unsplit (62 x U{478..3374} at 12:12 x 64, 744 workgroups: 85 us, split 94;
-// at 500 the two meet), as does one whose longest walk is at most 1,536 keys or barely more than a
-// chunk (the merge and the partial rows cost about 10 us). Measured, us, unsplit / chunk 256 /
+// workgroups per CU stays unsplit (62 x U{478..3374} at 12:12 x 64, 744 workgroups: 85 us, split 94),
+// as does one whose longest walk is at most 1,536 keys or barely more than a
+// chunk (the merge and the partial rows cost about 10 us), or that split_pays tells so. Measured, us, unsplit / chunk 256 /
 // 512 / 768 / 1,024 / 1,536, causal, by segments x keys, tails, heads x head_dim (the rule's choice):
 // (with the short pass and a plan; both are spared below)
 //   1 x 8,192, 1 row, 32:8 x 128                207 / 25 / 28 / 34 / 38 / 53        (256)
 //   4 x 4,096, 16 rows, 32:8 x 128              114 / 32 / 32 / 38 / 41 / 52        (320)
 //   16 x U{512..8192}, U{1..32}, 32:8 x 128     259 / 127 / 105 / 99 / 105 / 93     (1,408)
-//   64 x U{512..4096}, U{1..32}, 32:8 x 128     168 / 225 / 190 / 187 / 178 / 166   (1,536)
+//   64 x U{512..4096}, U{1..32}, 32:8 x 128     168 / 225 / 190 / 187 / 178 / 166   (unsplit)
 //   24 x U{600..2000}, U{1..16}, 32:8 x 128     76 / 56 / 51 / 46 / 45 / 55         (640)
 //   64 x U{512..8192}, U{1..16}, 8:2 x 256      381 / 160 / 141 / 135 / 147 / 130   (1,280)
 //   16 x U{512..8192}, U{1..32}, 12:12 x 64     138 / 70 / 67 / 67 / 69 / 68        (1,408)
@@ -546,6 +546,36 @@ constexpr size_t kSplitMaxBytes = (size_t)256 << 20;
 // of 384 keys for every segment took 97.6 us, 32 of 512 take 26.0, unsplit it is 42.7.
 int32_t longest_keys(const pe_attn_args *a) {
     return a->max_seqlen_k < a->total_tokens_k ? a->max_seqlen_k : a->total_tokens_k;
+}
+
+// Whether the split call is the faster one, by estimates (us) fitted to 3,200 calls timed both ways
+// (five head counts, 5 to 500 workgroups, 1 to 8 query tiles per segment, seven length distributions). The
+// unsplit call lasts as long as its longest walk (17, 30 or 40 ns a key by head_dim), but no less than
+// the keys take from memory (5.5 TB/s where they exceed the caches). The split call spreads all walks
+// over the chip (27, 30 or 52 ns a key with every slot taken) or streams the keys, and adds 6 us and
+// the partial rows, written and read back at 2.9 TB/s. Without the rule every call of up to two workgroups
+// per CU was split and 390 of the 3,200 got slower, unsplit / split: 62 x 4,000 keys, 16-row tails, 32:8 x
+// 128 181 / 247; 62 x 8,000, 128-row tails, 8:8 x 128 371 / 521. With it four do, by 5 % at most; one-row
+// tails at such sizes stay split: 64 x 4,096 keys, 32:8 x 128, 215 / 202. Two margins, each from 1,700 more
+// calls of which up to 30 got slower by 3 to 18 % without them:
+//  * A bound may be far above the longest segment. From three quarters of two workgroups per CU on, one
+//    past twice the mean counts as 1.4 times the mean (82 x U{1400..2500} keys, 96-row tails, 8:1 x 64
+//    under 16,384 59 / 69; 256 x U{100..300}, one row, 8:2 x 256 under 4,096 28 / 33). A call that does have
+//    such a segment then stays unsplit (240 x 100 keys and one of 4,096, 8:2 x 256, 148 / 47).
+//  * Chunks do not begin where windows do, so a windowed call has to gain a quarter (25 x U{500..8000}
+//    keys, 1,700 to the left, 96-row tails, 8:2 x 64 40 / 46).
+bool split_pays(const pe_attn_args *a, int64_t reach, int64_t longest, int64_t keys, int64_t chunk, int64_t groups,
+                int64_t slots) {
+    const double walk = a->head_dim == 64 ? 0.017 : a->head_dim == 128 ? 0.030 : 0.040;
+    const double busy = a->head_dim == 64 ? 0.027 : a->head_dim == 128 ? 0.030 : 0.052;
+    const double mean = (double)(keys < reach ? keys : reach);
+    const double walked = 2 * groups >= 3 * kCUs && reach > 2 * mean ? 1.4 * mean : (double)reach;
+    const double stream = mean * a->n_seq * a->n_heads_kv * a->head_dim * 4e-6;  // MB of keys and values
+    const double rows = (mean / chunk + 0.5) * a->total_tokens * a->n_heads_q;   // a row's chunks, on average
+    const double partial = rows * (a->head_dim + 2) * 4e-6;                      // MB
+    const double unsplit = walked * walk > stream / 5.5 ? walked * walk : stream / 5.5;
+    const double spread = mean * groups / slots * busy > stream / 6.0 ? mean * groups / slots * busy : stream / 6.0;
+    return 6.0 + spread + 0.7 * partial < (reach < longest ? 0.75 : 1.0) * unsplit;
 }
 
 Split split_of(const pe_attn_args *a, int g, int bm, int64_t cap) {
@@ -573,6 +603,7 @@ Split split_of(const pe_attn_args *a, int g, int bm, int64_t cap) {
     chunk = chunk < kSplitMinChunk ? kSplitMinChunk : chunk > kSplitMaxChunk ? kSplitMaxChunk : (chunk + 63) / 64 * 64;
     if (2 * reach < 3 * chunk) return s;
     const int chunks = (int)((longest + chunk - 1) / chunk);
+    if (!split_pays(a, reach, longest, keys, chunk, groups, slots)) return s;
     const size_t rows = (size_t)chunks * a->total_tokens * a->n_heads_q;
     if (chunks > 65535 || a->n_heads_q > 65535 || rows > kSplitMaxBytes / (4 * (a->head_dim + 2))) return s;
     s.chunk = (int)chunk;
