@@ -98,7 +98,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     if (WIN && !SPLIT && p.wl >= 0 && p.wr >= 0) {
         const int rh = kXcdRun * p.hgroups;
         const int j = (int)(blockIdx.x >> 3);
-        item = ((j / rh) * 8 + (int)(blockIdx.x & 7)) * rh + j % rh;
+        // Without a plan the tiles come in batch order: each round of runs begins one XCD further, or equal
+        // segments of as many tiles as divide a round would send all their cheap tiles (the first ones of a
+        // causal segment) to the same XCDs. Causal with 256 keys to the left, planned / without / with, us:
+        // 180 x 256 tokens, 32:8 heads 137 / 150 / 135; 128 x 256, 16:2 heads 53 / 54 / 47; 64 x 512, 32:8
+        // heads 121 / 131 / 120.
+        const int xcd = DIRECT ? (int)((blockIdx.x + j / rh) & 7) : (int)(blockIdx.x & 7);
+        item = ((j / rh) * 8 + xcd) * rh + j % rh;
     }
     int entry = item / p.hgroups;
     int hg = item - entry * p.hgroups;
