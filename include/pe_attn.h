@@ -156,7 +156,10 @@ int pe_attn_key_chunks(const pe_attn_args *args);
 
 /* Packed varlen attention, both kernels in one call. Segments are routed per segment on the
    device by their length (no host read of cu_seqlens): short ones to the LDS-resident kernel,
-   long ones through a device-built, cost-ordered tile list to the tiled MFMA kernel.
+   long ones through a device-built, cost-ordered tile list to the tiled MFMA kernel, or, in
+   narrow-window calls and small split ones, through tiles that every workgroup finds for itself. Such
+   a call leaves the list's place in the workspace unwritten: only pe_attn_plan makes a plan for
+   pe_attn_tiled_fwd to read.
    Replaces the reference's FlashAttention varlen leg (packed_encoders/ops.py:432-461,
    ops.py:521-532) and the varlen candidates of select_attention
    (packed_encoders/runtime/attention.py:66-126), GQA, causal, window and the fused sigmoid
@@ -179,7 +182,7 @@ int pe_varlen_attn_fwd(const pe_attn_args *args, void *workspace, size_t workspa
 #define PE_ATTN_STATIC_SCRATCH_BYTES (1u << 20)
 int pe_varlen_attn_fwd_noalloc(const pe_attn_args *args, hipStream_t stream);
 
-/* The three stages pe_varlen_attn_fwd runs, for callers that reuse one plan across calls
+/* The three stages of a planned, unsplit pe_varlen_attn_fwd, for callers that reuse one plan across calls
    (the 22 layers of a packed forward share cu_seqlens: one plan per window kind serves all
    of them) or time one kernel. A plan is valid for arguments with the same cu_seqlens
    contents, n_seq, total_tokens, max_seqlen, min_seqlen, head counts, window, causal and

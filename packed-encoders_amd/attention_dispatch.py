@@ -13,7 +13,8 @@ The rule, fitted to the short-vs-tiled sweep (``python bench.py --dispatch-sweep
 profiles/dispatch_sweep.md and re-derived by ``fit_boundary`` in the tests):
 
 - ``max_seqlen <= 128``: every segment takes the short kernel, at its smallest key capacity
-  (32, 64 or 128) that holds ``max_seqlen`` — faster than the tiled kernel at every measured
+  (32, 64 or 128; a call of 65 to 96 tokens launches the kernel with 96 keys, which the
+  sweep did not have) that holds ``max_seqlen`` — faster than the tiled kernel at every measured
   length, both head dims and both batch scales (the reference's Triton kernel likewise keys its
   tile choice on ``Smax``, triton_packed_attention.py:29-42);
 - longer batches: segments up to the fitted boundary (64 for head_dim 64, 32 for head_dim 128)
@@ -40,7 +41,7 @@ from typing import Iterable, Mapping, Sequence
 
 import torch
 
-SHORT_CAPACITIES = (32, 64, 128)  # key capacities of the short kernel's LDS tiles
+SHORT_CAPACITIES = (32, 64, 128)  # key capacities of the short kernel's LDS tiles in the sweep's table
 SHORT_HEAD_DIMS = (64, 128)       # head dims the short kernel serves
 
 

@@ -239,8 +239,9 @@ int launch_short_t(const AttnParams &p, hipStream_t stream) {
 // Compute units of an MI355X.
 constexpr int64_t kCUs = 256;
 
-// Static short-kernel choice: key capacity SK (32/64/128) and heads per workgroup, sized so
-// the workgroup's K and V^T stay within ~75 KB of LDS (two workgroups per CU).
+// Static short-kernel choice (pe_attn_short_config): key capacity SK (32/64/128) and heads per
+// workgroup, sized so the workgroup's K and V^T stay within ~75 KB of LDS (two workgroups per CU).
+// short_launch_shape refines it for a call.
 void short_shape(int max_len, int d, int *sk, int *hpw) {
     *sk = max_len <= 32 ? 32 : (max_len <= 64 ? 64 : 128);
     if (d == 64)
@@ -445,11 +446,11 @@ int launch_split_d(const AttnParams &p, int g, int bm, int64_t cap, int chunks, 
 // Whether a call runs without a plan: a narrow two-sided window (full tiles cost about the same in any
 // order; at +-600 that no longer holds and the longest-first plan is as good) in the tiled kernel,
 // over at most kDirectSegments segments. The plan kernel takes 5 to 9 us of such a call, finding a
-// tile from cu_seqlens about what reading its work entry takes. Calls with and without the plan, us,
-// 12 heads, +-64: 64 documents of median 400 tokens (300 tiles) 63.4 -> 59.5, 8 documents 21.0 -> 13.0,
-// 1 x 3,000 20.7 -> 12.7, 256 x median 300 174.5 -> 163.4; 64 documents causal with 256 keys to the left
-// 65.1 -> 60.3. 16 x 8,192 at 16 heads (16,384 tiles x heads) 237.3 -> 240.6, so the largest calls keep
-// it. The staged entry points do too: layers share their plan.
+// tile from cu_seqlens about what reading its work entry takes. Calls with and without the plan, us, both
+// in one build, 12 heads, +-64: 64 documents of median 400 tokens (30,894 in all) 54.0 -> 47.5, 8 documents
+// 21.4 -> 13.2, 1 x 3,000 21.1 -> 12.7, 256 x median 300 143.4 -> 136.5; 64 documents causal with 256 keys
+// to the left 60.7 -> 53.7. 16 x 8,192 at 16 heads (16,384 tiles x heads) 240.0 -> 246.7, so the largest
+// calls keep it. The staged entry points do too: layers share their plan.
 constexpr int kDirectWindow = 256;
 constexpr int64_t kDirectMaxTiles = 12288;
 bool plans_itself(const pe_attn_args *a) {

@@ -2,9 +2,9 @@
 // one decoded token to a short tail). A workgroup of the tiled kernels walks its tile's keys
 // one after another, so such a call fills a fraction of the chip and lasts as long as its longest
 // segment: 16 segments of up to 8,192 keys at 32:8 heads of 128 were 128 workgroups and 128 serial
-// key tiles, the call 244 us for 327 MB. Split, a workgroup takes one chunk of the keys (grid y)
+// key tiles, the call 245 us for 327 MB. Split, a workgroup takes one chunk of the keys (grid y)
 // and writes its unnormalised rows with their maximum and sum in fp32, and merge_kernel adds the
-// chunks of a row: 92 us (3.6 TB/s). split_of (pe_attn_capi.hip) holds the rule and its figures.
+// chunks of a row: 89 us (3.7 TB/s). split_of (pe_attn_capi.hip) holds the rule and its figures.
 //
 // The tiled kernels take SPLIT as a template flag: same loads, products and softmax over the
 // chunk, one query tile per work entry, partial rows instead of the epilogue. A row whose tile

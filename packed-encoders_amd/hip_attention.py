@@ -460,7 +460,9 @@ def select_packed_short_attention_config(max_seqlen: int, head_dim: int = 64) ->
     ``num_stages`` staging passes (one: every load is issued before a single wait). The extra
     keys describe this kernel's tiles. Like the reference, any ``max_seqlen`` gets an answer:
     lengths past 128 report the 128-key shape, the largest the short kernel has (such batches
-    run the tiled kernel for their longer segments)."""
+    run the tiled kernel for their longer segments). A launch may refine the table for its batch
+    (96 of the 128 keys for segments of 65 to 96, fewer heads for small batches and with RoPE
+    tables): ``pe_attn_kernels`` reports launches."""
     smax = min(max(int(max_seqlen), 1), 128)
     out = (ctypes.c_int32 * 4)()
     _lib.check(_lib.library().pe_attn_short_config(smax, int(head_dim), out), "pe_attn_short_config")
