@@ -136,8 +136,8 @@ def useful_flops_served(workload, short_max, kernel):
 def kernel_instance(lib, call, workload):
     """The name rocprofv3 lists (template arguments included) for the kernels of one layer's
     call, as the library reports its choice (pe_attn_kernels): (short kernel, long kernel). LayerCall
-    launches the stages over a shared plan, so its long kernel is the unsplit, planned instance (the
-    last two arguments false)."""
+    launches the stages over a shared plan and without RoPE tables, so its long kernel is the unsplit,
+    planned instance (the last two arguments false), its short kernel the one without RoPE."""
     from packed_encoders_amd import _lib
 
     out = (ctypes.c_int32 * 6)()
@@ -150,7 +150,7 @@ def kernel_instance(lib, call, workload):
     g = math.gcd(workload.n_heads_q // workload.n_heads_kv, 4)
     short = None
     if out[0]:
-        short = f"pe::short_attn_kernel<{d}, {out[0]}, {out[4]}, {gate}>"
+        short = f"pe::short_attn_kernel<{d}, {out[0]}, {out[4]}, {gate}, false>"
     long = {
         _lib.KERNEL_NONE: None,
         _lib.KERNEL_TILED: f"pe::tiled_attn_kernel<64, {g}, 64, 3, {gate}, {win}, false, false>",

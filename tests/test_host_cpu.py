@@ -540,3 +540,28 @@ def test_pack_validation_gate_on_cpu():
     assert report.pieces["attention"].max_abs_error is not None
     assert report.pieces["attention_bshd"].skipped_reason
     pe.unpack(m)
+
+
+@pytest.mark.parametrize("name", ["C1", "Q4096", "C2", "C4-band", "C5"])
+def test_bench_names_the_kernels_that_the_profiles_list(name):
+    """bench.kernel_instance gives the name under which the committed traffic table holds the workload's
+    dominant kernel (rocprofv3's, template arguments included), so the bench line finds it."""
+    import ctypes
+    import json
+    from types import SimpleNamespace
+
+    import bench
+    from packed_encoders_amd import _lib
+
+    w = bench.WORKLOADS[name]()
+    short_max = attention_dispatch.hip_short_max(w.head_dim, max_seqlen=w.max_seqlen)
+    stage, _, layers = bench.dominant(w, short_max)
+    layer = w.layers[layers[0]]
+    a = _lib.AttnArgs()
+    a.struct_size, a.dtype = ctypes.sizeof(_lib.AttnArgs), 1
+    a.n_seq, a.total_tokens, a.max_seqlen, a.min_seqlen = len(w.lengths), w.total_tokens, w.max_seqlen, min(w.lengths)
+    a.n_heads_q, a.n_heads_kv, a.head_dim, a.softmax_scale = w.n_heads_q, w.n_heads_kv, w.head_dim, w.scale
+    a.window_left, a.window_right, a.causal, a.short_max = *layer.window, int(layer.causal), short_max
+    names = bench.kernel_instance(_lib.library(), SimpleNamespace(args=a, layer=layer), w)
+    table = json.loads((bench.ROOT / "profiles" / "traffic.json").read_text())["kernels"]
+    assert f"{w.name}:{names[0 if stage == 'short' else 1]}" in table
