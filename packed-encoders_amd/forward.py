@@ -334,13 +334,17 @@ def packed_forward(model: nn.Module, params: ModernBertParams, packed_ids: Tenso
 
 def packed_core(model: nn.Module, params: ModernBertParams, x: Tensor, cu_seqlens: Tensor, max_seqlen: int,
                 position_ids: Tensor, *, execution, min_seqlen: int = 0) -> Tensor:
-    """RoPE tables per token (positions below ``max_seqlen``), then ``core`` on ``[1, T, hidden]``
-    with the HIP backend. Shared by the eager packed forward and the graph runner's capture."""
+    """RoPE tables per token, then ``core`` on ``[1, T, hidden]`` with the HIP backend. Shared by the
+    eager packed forward and the graph runner's capture.
+
+    Positions lie below ``max_seqlen`` or, as the columns that ``unpad`` gives a mask padding on the left,
+    within the model's ``max_position_embeddings``; others get NaN tables."""
     device, dtype, d = x.device, x.dtype, params.head_dim
+    table = max(int(max_seqlen), int(getattr(getattr(model, "config", None), "max_position_embeddings", 0) or 0))
 
     def rows(theta: float) -> tuple[Tensor, Tensor]:
         if execution.rope_tables is ops.rope_tables:
-            return ops.rope_rows(position_ids, max_seqlen, d, theta, dtype)
+            return ops.rope_rows(position_ids, table, d, theta, dtype)
         return tuple(t[0].index_select(0, position_ids)[None]
                      for t in execution.rope_tables(max_seqlen, d, theta, device, dtype))
 

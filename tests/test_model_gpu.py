@@ -101,6 +101,38 @@ def test_pack_hip_validates_and_matches_hf_fp32(pe, monkeypatch):
     pe.unpack(model)
 
 
+@pytest.mark.parametrize("graphs", [False, True], ids=["eager", "graph"])
+def test_left_padded_batches_match_hf_fp32(pe, graphs):
+    """A mask that pads on the left puts positions (columns) past the longest length: the tokens get those
+    columns' rotations, as Hugging Face's forward gives them, eagerly and replayed. Positions outside the
+    model's range give NaN, never a rotation."""
+    from packed_encoders_amd import forward
+
+    announce(f"left-padded batch, graphs {graphs}")
+    ref = make_model().cuda()
+    model = copy.deepcopy(ref).to(torch.bfloat16)
+    ids, mask = batch([300, 100, 37], seed=5)
+    ids = torch.nn.functional.pad(ids, (150, 0))  # every row's tokens end or lie past column 300
+    mask = torch.nn.functional.pad(mask, (150, 0))
+    config = pe.GraphConfig(max_batch=8, max_seq=512, pad_to=64, warmup=2)
+    pe.pack(model, attention_backend="hip", validate=False, **({"cuda_graph": config} if graphs else {}))
+    live = mask.bool()
+    with torch.no_grad():
+        want = ref(input_ids=ids, attention_mask=mask).last_hidden_state
+        for _ in range(3 if graphs else 1):
+            got = model(input_ids=ids, attention_mask=mask).last_hidden_state
+            cos = token_cosine(got[live], want[live])
+            assert cos.min() >= 0.995 and cos.mean() >= 0.999, (cos.min(), cos.mean())
+        flat, _, cu, max_seqlen, positions = forward.unpad(ids, mask)
+        assert int(positions.max()) >= max_seqlen
+        positions[7] = -1  # in the first segment
+        bad = forward.packed_forward(model, pe.config.ModernBertParams.from_hf_config(model.config), flat, cu, max_seqlen,
+                                     positions, backend="hip", _allow_graph=graphs)
+        first = slice(0, int(cu[1]))
+        assert bad[7].isnan().all() and not bad[first.stop:].isnan().any()
+    pe.unpack(model)
+
+
 def test_packed_forward_hip_matches_dense_fallback(pe):
     from packed_encoders_amd import forward
 
