@@ -165,7 +165,7 @@ def test_other_threads_run_during_a_launch(pe, name):
         try:
             thread.start()
             before, outs = ran[0], []
-            while ran[0] == before and len(outs) < 4000:
+            while ran[0] == before and len(outs) < 20000:
                 outs.append(call())
             during = ran[0] - before
         finally:
